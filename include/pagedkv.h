@@ -149,8 +149,9 @@ int pkv_decode_fast_path(int32_t n_heads, int32_t n_kv_heads, int32_t head_dim,
  * path only). Pass NULL for all three otherwise.
  *
  * Geometries outside the fast kernel (head_dim not 64/128, more than 16
- * query heads per KV head, page_size != 16, fp32) run the generic kernel,
- * which reads kv_indptr / kv_indices / kv_lens instead of the plan.
+ * query heads per KV head, page_size != 16, fp32) read kv_indptr /
+ * kv_indices / kv_lens instead of the plan: fp32 at head_dim 64/128 and
+ * page_size 16 on its own matrix-core kernel, the rest on the generic one.
  */
 int pkv_attend_decode(const void* q, void* out,
                       void* k_pool, void* v_pool, int64_t num_blocks,
@@ -204,8 +205,10 @@ int pkv_plan_prefill(const int32_t* cu_query_lens, const int32_t* kv_indptr,
 /*
  * Query tile (tokens per plan tile) for which pkv_attend_prefill runs its
  * matrix-core kernel on this geometry: 128 / (n_heads / n_kv_heads), so a
- * tile is 128 query rows of one KV head. 0 if the geometry has no such
- * kernel (any q_tile then runs the generic kernel). Counterpart of the
+ * tile is 128 query rows of one KV head; for fp32, 32 / (n_heads /
+ * n_kv_heads), at least 1 (its kernel takes any q_tile, this one without
+ * idle workgroups). 0 if the geometry has no such kernel (any q_tile then
+ * runs the generic kernel). Counterpart of the
  * tile choice inside FlashInfer's prefill plan
  * (serving/backends/flashinfer_backend.py:635-649).
  */
@@ -222,8 +225,10 @@ int pkv_prefill_q_tile(int32_t n_heads, int32_t n_kv_heads, int32_t head_dim,
  * causal). q, out: [n_tokens, n_heads, head_dim]. `batch_indices` maps each
  * token to its sequence. `plan` is the device copy of pkv_plan_prefill's
  * output (q_tile must match the one given to the plan). The matrix-core
- * kernel runs when q_tile == pkv_prefill_q_tile(...) != 0; otherwise the
- * generic kernel runs (it reads cu_query_lens / batch_indices, not the plan).
+ * kernel runs when q_tile == pkv_prefill_q_tile(...) != 0 (fp32: any q_tile,
+ * with 16-byte aligned q, out and pools); otherwise the generic kernel runs
+ * (it reads cu_query_lens / batch_indices, not the plan; fp32 without a plan
+ * too).
  */
 int pkv_attend_prefill(const void* q, void* out,
                        const void* k_pool, const void* v_pool, int64_t num_blocks,

@@ -3,8 +3,9 @@
 // the fast kernels do not cover.
 //
 //  * generic_kernel — any geometry, any query length, bottom-right causal;
-//    used when prefill.hip's MFMA kernel does not cover the geometry or the
-//    plan was tiled for another query tile.
+//    used when neither prefill.hip's MFMA kernel nor, for fp32 pools,
+//    attention_f32.hip's covers the geometry, or the plan was tiled for
+//    another query tile.
 //
 // Numerics follow serving/backends/paged_torch.py:443-485: scores and
 // softmax in fp32, probabilities rounded to the pool dtype, PV accumulated
@@ -22,6 +23,12 @@ int run_fast_prefill(const void* q, void* out, const void* kp, const void* vp, i
                      int32_t page_size, float scale, int32_t dtype, const int32_t* plan,
                      int32_t n_tiles, int32_t q_tile, int32_t* status, hipStream_t s,
                      bool* ran);
+
+int run_f32(const void* q, void* out, const void* kp, const void* vp, int64_t nb,
+            const int32_t* cu_q, const int32_t* indptr, const int32_t* indices,
+            const int32_t* kv_lens, int32_t Hq, int32_t Hkv, int32_t D, int32_t page_size,
+            float scale, const int32_t* plan, int32_t n_tiles, int32_t q_tile, int32_t* status,
+            hipStream_t s, bool* ran);
 
 // ------------------------------------------------------------------ plans ---
 
@@ -209,6 +216,10 @@ int generic_decode(const void* q, void* out, const void* kp, const void* vp, int
   if (dtype == PKV_DTYPE_BF16)
     return launch_generic<__bf16>(q, out, kp, vp, nb, nullptr, indptr, indices, kv_lens,
                                   nullptr, n_seqs, n_seqs, Hq, Hkv, D, ps, scale, status, s);
+  bool ran = false;
+  const int rc = run_f32(q, out, kp, vp, nb, nullptr, indptr, indices, kv_lens, Hq, Hkv, D, ps,
+                         scale, nullptr, n_seqs, 1, status, s, &ran);
+  if (rc || ran) return rc;
   return launch_generic<float>(q, out, kp, vp, nb, nullptr, indptr, indices, kv_lens, nullptr,
                                n_seqs, n_seqs, Hq, Hkv, D, ps, scale, status, s);
 }
@@ -236,5 +247,11 @@ extern "C" int pkv_attend_prefill(const void* q, void* out, const void* k_pool,
     return launch_generic<_Float16>(q, out, k_pool, v_pool, num_blocks, cu_query_lens, kv_indptr, kv_indices, kv_lens, batch_indices, n_seqs, n_tokens, n_heads, n_kv_heads, head_dim, page_size, scale, status_word, s);
   if (dtype == PKV_DTYPE_BF16)
     return launch_generic<__bf16>(q, out, k_pool, v_pool, num_blocks, cu_query_lens, kv_indptr, kv_indices, kv_lens, batch_indices, n_seqs, n_tokens, n_heads, n_kv_heads, head_dim, page_size, scale, status_word, s);
+  if (plan) {
+    rc = run_f32(q, out, k_pool, v_pool, num_blocks, cu_query_lens, kv_indptr, kv_indices,
+                 kv_lens, n_heads, n_kv_heads, head_dim, page_size, scale, plan, n_tiles, q_tile,
+                 status_word, s, &ran);
+    if (rc || ran) return rc;
+  }
   return launch_generic<float>(q, out, k_pool, v_pool, num_blocks, cu_query_lens, kv_indptr, kv_indices, kv_lens, batch_indices, n_seqs, n_tokens, n_heads, n_kv_heads, head_dim, page_size, scale, status_word, s);
 }

@@ -424,6 +424,8 @@ static PrefillFn prefill_d(int D, int G) {
   }
 }
 
+int f32_q_tile(int32_t Hq, int32_t Hkv, int32_t D, int32_t page_size);  // attention_f32.hip
+
 // The MFMA prefill kernel for this geometry, or null (generic kernel).
 PrefillFn fast_prefill(int32_t dtype, int32_t Hq, int32_t Hkv, int32_t D, int32_t page_size) {
   if (page_size != 16 || Hkv <= 0 || Hq % Hkv) return nullptr;
@@ -439,8 +441,9 @@ using namespace pkv;
 
 extern "C" int pkv_prefill_q_tile(int32_t n_heads, int32_t n_kv_heads, int32_t head_dim,
                                   int32_t page_size, int32_t dtype) {
-  if (!fast_prefill(dtype, n_heads, n_kv_heads, head_dim, page_size)) return 0;
-  return kPrefillRows / (n_heads / n_kv_heads);
+  if (fast_prefill(dtype, n_heads, n_kv_heads, head_dim, page_size))
+    return kPrefillRows / (n_heads / n_kv_heads);
+  return dtype == PKV_DTYPE_F32 ? f32_q_tile(n_heads, n_kv_heads, head_dim, page_size) : 0;
 }
 
 namespace pkv {
