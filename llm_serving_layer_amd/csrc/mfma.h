@@ -63,4 +63,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t ws_rsrc(void* base, uint32_t b
   return __builtin_amdgcn_make_buffer_rsrc(base, (short)0, (int)bytes, 0x00020000);
 }
 
+// Row `row` of a tile stores its 16-byte chunk c at chunk position
+// c ^ xr(row), xr a permutation of row & 7. Eight consecutive rows reading
+// the same chunk (the K operand reads) then hit eight different chunk
+// positions, and so do four consecutive rows reading chunks 2j and 2j + 1
+// (the transposed V reads): both are free of bank conflicts.
+__device__ __forceinline__ int xr(int row) { return ((row & 3) << 1) | ((row >> 2) & 1); }
+// Byte offset of element `e` (of 2-byte elements) in row `row` of a tile.
+template <int RB>
+__device__ __forceinline__ int swz(int row, int e) {
+  return row * RB + ((((e >> 3) ^ xr(row)) & 7) | ((e >> 3) & ~7)) * 16 + (e & 7) * 2;
+}
+
 }  // namespace pkv

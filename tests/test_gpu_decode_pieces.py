@@ -1,0 +1,72 @@
+"""
+The two decode kernels (csrc/decode.hip) give one result: a sequence's output
+has the same bits whether its batch is small (a workgroup per piece and KV
+head) or large (bins of pieces streamed by resident workgroups), with the
+step's rows appended inside the launch, at the sizes where the small-batch
+kernel can go wrong: one row, page edges, the pages its four waves share, its
+chunks of 20 pages and their remainders, every group size, and non-finite
+values in the unused rows of a last page.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from llm_serving_layer_amd import BlockAllocator, SequenceBlocks
+from llm_serving_layer_amd.backend import MI355XBackend
+
+from ._util import grow_and_assemble
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# history tokens; the step appends one more: whole sequences (17 pages), cut
+# ones (with and without a folded tail), and with part_pages=64 chunks of 20
+EDGES = [0, 1, 14, 15, 16, 17, 31, 63, 64, 79, 80, 255, 270, 271, 272, 303, 304, 319, 320, 335,
+         336, 543, 640, 660, 1023, 1071]
+
+
+@pytest.mark.parametrize("n_heads, d, dtype, part_pages", [
+    (1, 64, torch.float16, 17), (2, 128, torch.float16, 17), (4, 64, torch.bfloat16, 17),
+    (8, 128, torch.bfloat16, 17), (16, 64, torch.float16, 17), (16, 128, torch.float16, 64),
+    (4, 64, torch.float16, 64)])
+def test_small_and_large_batches_give_the_same_bits(n_heads, d, dtype, part_pages):
+    print(f"decode pieces heads={n_heads} d={d} {dtype} part_pages={part_pages}", flush=True)
+    lens = (EDGES * 12)[:300]          # 300 pieces or more: the streaming kernel
+    nb = sum(n // 16 + 1 for n in lens)
+    alloc = BlockAllocator(nb, 16)
+    seqs = [SequenceBlocks(alloc, seq_id=i) for i in range(len(lens))]
+    for s, n in zip(seqs, lens):
+        s.append(n)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rand = lambda *s: torch.randn(s, generator=g, device=DEV).to(dtype)  # noqa: E731
+    big, few = [MI355XBackend(1, nb, 16, 1, n_heads, d, device=DEV, dtype=dtype,
+                              part_pages=part_pages) for _ in range(2)]
+    k, v = rand(nb, 16, 1, d), rand(nb, 16, 1, d)
+    for s, n in zip(seqs, lens):       # rows past the history hold no numbers
+        if n % 16:
+            k[s.block_ids[-1], n % 16:] = float("nan")
+            v[s.block_ids[-1], n % 16:] = float("inf")
+    for bk in (big, few):
+        bk.k_pool[0].copy_(k)
+        bk.v_pool[0].copy_(v)
+    q = 2.0 * rand(len(lens), n_heads, d)   # scores wide enough to move the reference
+    kn, vn = rand(len(lens), 1, d), rand(len(lens), 1, d)
+    meta = grow_and_assemble(seqs, [1] * len(lens), 16, device=DEV)
+    big.append_kv(0, kn, vn, meta)
+    want = big.attend(q, 0, d ** -0.5, meta)
+    assert big._planned.n_work >= 256
+    assert torch.isfinite(want).all()
+    for at in range(0, len(lens), 26):
+        part = slice(at, min(at + 26, len(lens)))
+        for s in seqs[part]:           # the step's token again, in a batch of its own
+            s.num_tokens -= 1
+        meta = grow_and_assemble(seqs[part], [1] * len(seqs[part]), 16, device=DEV)
+        few.append_kv(0, kn[part], vn[part], meta)
+        got = few.attend(q[part], 0, d ** -0.5, meta)
+        assert few._planned.n_work < 256
+        assert torch.equal(got, want[part]), f"sequences from {at}"
+    assert torch.equal(few.k_pool[0].view(torch.int16), big.k_pool[0].view(torch.int16))
+    assert torch.equal(few.v_pool[0].view(torch.int16), big.v_pool[0].view(torch.int16))
+    big.check_device_errors()
+    few.check_device_errors()
