@@ -10,9 +10,9 @@
 //
 // The KV axis is walked 32 tokens (two pages) at a time. A tile of K and of
 // V (those rows x head_dim of head h) goes straight from memory into one of
-// four LDS buffers (a ring; direct-to-LDS buffer loads two tiles ahead,
-// rows unpadded with their 16-byte chunks swizzled) and is read by every
-// wave. All products are 32x32x16 MFMAs, so every LDS byte read feeds 32
+// four LDS buffers (a ring; direct-to-LDS buffer loads two tiles ahead, each
+// wave one page of one tensor, rows unpadded with their 16-byte chunks
+// swizzled) and is read by every wave. All products are 32x32x16 MFMAs, so every LDS byte read feeds 32
 // query rows:
 //  * S^T = K Q^T: K rows from LDS as the A operand, Q^T held in registers
 //    as the B operand. Lane (row n, group g) gets 16 scores of its query row
@@ -55,14 +55,13 @@ template <> struct Mma32<__bf16> {
   }
 };
 
-// LDS of one workgroup: a ring of four K/V tile buffers, each its own
-// variable (so the compiler's wait before a tile read covers only the loads
-// into that buffer), rows unpadded with 16-byte chunks XOR-swizzled by row.
+// LDS of one workgroup: a ring of four K/V tile buffers, rows unpadded with
+// 16-byte chunks XOR-swizzled by row.
 template <typename T, int D> struct PrefillLds {
   static constexpr int TT = 32;                        // KV tokens per tile
   static constexpr int RB = D * (int)sizeof(T);        // bytes of one head's row
   static constexpr int TILE = TT * RB;                 // one K (or V) tile
-  static constexpr int LPT = TILE / (kPrefillThreads * 16);  // 16-byte loads per thread
+  static constexpr int LPT = TILE / 2 / 1024;          // wave loads of a page of one tensor
 };
 
 template <typename T, int D, int G>
@@ -83,7 +82,6 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(
   constexpr int RB = L::RB;
   constexpr int CPR = RB / 16;           // 16-byte chunks per row
   constexpr int LPT = L::LPT;
-  static_assert(LPT >= 1 && L::TILE == LPT * kPrefillThreads * 16, "whole 1 KiB wave loads");
   static_assert(64 % CPR == 0 && PS % (64 / CPR) == 0, "a wave load stays in one page");
   __shared__ __align__(16) unsigned char buf0[2 * L::TILE];
   __shared__ __align__(16) unsigned char buf1[2 * L::TILE];
@@ -123,60 +121,46 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(
     }
   }
 
-  // Tiles past the end and rows at or past kv_len are outside their buffer
-  // ranges: nothing is read for them. The ring starts zeroed, so what such
-  // rows hold in LDS is finite and only ever meets zero probabilities.
-  for (int i = tid; i < 2 * L::TILE / 16; i += kPrefillThreads) {
-    reinterpret_cast<u32x4*>(buf0)[i] = u32x4{0u, 0u, 0u, 0u};
-    reinterpret_cast<u32x4*>(buf1)[i] = u32x4{0u, 0u, 0u, 0u};
-    reinterpret_cast<u32x4*>(buf2)[i] = u32x4{0u, 0u, 0u, 0u};
-    reinterpret_cast<u32x4*>(buf3)[i] = u32x4{0u, 0u, 0u, 0u};
-  }
-
-  // Load k of a tile covers 64 x 16 bytes = 64 / CPR consecutive rows, all in
-  // one page: its page id is wave-uniform, read with a scalar load a tile
-  // ahead. (Scalar loads, so the vector-memory count holds tile loads only:
-  // a plain vector load may complete before a direct-to-LDS load issued
-  // earlier, so the count cannot prove a tile landed if the two mix.)
+  // A wave loads one page of one tensor of a tile, 16 rows of the KV head: one
+  // buffer range to set up instead of one per page and tensor (about 45 scalar
+  // instructions a step instead of 130; a 777-token prompt, head_dim 128, 8
+  // layers with their appends: 205 -> 195 us, with the ring no longer zeroed
+  // at the start; no change where four waves share a SIMD). The page id is
+  // read with a scalar load a tile ahead. (Scalar loads, so the vector-memory count holds
+  // tile loads only: a plain vector load may complete before a direct-to-LDS
+  // load issued earlier, so the count cannot prove a tile landed if the two
+  // mix.)
   const int npages = (kv_len + PS - 1) / PS;
   const uint32_t rowbytes = (uint32_t)(row * sizeof(T));
+  const uint32_t pagebytes = PS * rowbytes;
   // ids at or past this are out of range (kv_indices entries are int32)
   const uint32_t nb32 = num_blocks > 0x7fffffffLL ? 0x80000000u : (uint32_t)num_blocks;
-  static_assert(TT % PS == 0, "a tile starts at a page boundary");
-  auto page_of = [&](int t, int k) { return (t * TT + ((k * 4 + wave) * 64) / CPR) / PS; };
-  auto load_ids = [&](int t, int* ids) {   // this wave's page ids for tile t
+  static_assert(TT == 2 * PS, "a tile is two pages");
+  const int wpage = wave & 1;
+  const T* const wpool = wave < 2 ? kpool : vpool;
+  const uint32_t wdst = (wave < 2 ? 0 : L::TILE) + wpage * PS * RB;
+  constexpr int RPI = 64 / CPR;                  // rows of a wave load
+  uint32_t voff[LPT];
 #pragma unroll
-    for (int k = 0; k < LPT; ++k) {
-      const int pg = min(page_of(t, k), npages - 1);
-      ids[k] = __builtin_amdgcn_readfirstlane(kv_indices[pbase + pg]);
-    }
+  for (int k = 0; k < LPT; ++k) {                // (rows k * RPI: in the scalar offset)
+    const int lc = ((lane % CPR) ^ xr(k * RPI + lane / CPR)) & 7 | ((lane % CPR) & ~7);
+    voff[k] = (uint32_t)(lane / CPR) * rowbytes + (uint32_t)(h * RB + lc * 16);
+  }
+  auto load_id = [&](int t) {   // this wave's page id for tile t
+    return __builtin_amdgcn_readfirstlane(kv_indices[pbase + min(2 * t + wpage, npages - 1)]);
   };
-  auto load_tile = [&](int t, const int* ids, unsigned char* dst) {
-#pragma unroll
-    for (int k = 0; k < LPT; ++k) {
-      const int c0 = (k * 4 + wave) * 64;            // first chunk of this wave load
-      const int row0 = c0 / CPR;
-      const int pg = page_of(t, k);
-      const int raw = ids[k];
-      const bool bad = (uint32_t)raw >= nb32;   // (negative ids too)
-      if (bad && pg < npages && lane == 0) flag(status, PKV_STATUS_BAD_PAGE);
-      const int live_rows = bad ? 0 : min(PS, kv_len - pg * PS);   // <= 0 past the end
-      const int64_t pid = bad ? 0 : raw;
-      const uint32_t range = live_rows > 0 ? (uint32_t)live_rows * rowbytes : 0u;
-      const __amdgpu_buffer_rsrc_t rk =
-          ws_rsrc(const_cast<T*>(kpool) + pid * PS * row, range);
-      const __amdgpu_buffer_rsrc_t rv =
-          ws_rsrc(const_cast<T*>(vpool) + pid * PS * row, range);
-      const int rr = row0 + lane / CPR;              // the lane's row of the tile
-      const int lc = (((lane % CPR) ^ xr(rr)) & 7) | ((lane % CPR) & ~7);  // its chunk
-      // (a tile starts at a page boundary: the row within its page is rr % PS)
-      const uint32_t off = (uint32_t)(rr % PS) * rowbytes + (uint32_t)(h * RB + lc * 16);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rk, (__attribute__((address_space(3))) void*)(dst + c0 * 16), 16, off, 0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rv, (__attribute__((address_space(3))) void*)(dst + L::TILE + c0 * 16), 16, off, 0,
-          0, 0);
-    }
+  // Rows past kv_len, pages past the last and out-of-range pages are outside
+  // the buffer range: zeros land in LDS without a memory access.
+  auto load_tile = [&](int t, int raw, const unsigned char* dst) {
+    const int pg = 2 * t + wpage;
+    const bool bad = (uint32_t)raw >= nb32;   // (negative ids too)
+    if (bad && pg < npages && lane == 0) flag(status, PKV_STATUS_BAD_PAGE);
+    const int live_rows = bad ? 0 : min(PS, kv_len - pg * PS);   // <= 0 past the end
+    const uint32_t pid = bad ? 0u : (uint32_t)raw;
+    load_to_lds<LPT>(
+        raw_rsrc(reinterpret_cast<const char*>(wpool) + (uint64_t)pid * pagebytes,
+                 live_rows > 0 ? (uint32_t)live_rows * rowbytes : 0u),
+        voff, RPI * rowbytes, lds_address(dst) + wdst);
   };
 
   // O^T accumulators: o[dh][rr] = O[row][32 dh + 8 (rr / 4) + 4 g + rr % 4].
@@ -321,38 +305,47 @@ __global__ __launch_bounds__(kPrefillThreads) void prefill_kernel(
   // whose PV ran in the previous step), loads the pages of tile t + 2,
   // computes tile t beside the PV of tile t - 1, and loads the page ids of
   // tile t + 3.
-  int ids0[LPT], ids1[LPT], ids2[LPT], ids3[LPT];   // page ids of tile j in ids(j % 4)
-  load_ids(0, ids0);
-  load_ids(1, ids1);
-  __syncthreads();   // the zeroed ring before any load lands in it
-  load_tile(0, ids0, buf0);
-  load_ids(2, ids2);
-  load_tile(1, ids1, buf1);
+  // The first step's PV meets zero probabilities in buf3, which no tile has
+  // filled yet: zeros there (visible to every wave at the step's barrier).
+  for (int i = tid; i < L::TILE / 16; i += kPrefillThreads)
+    reinterpret_cast<u32x4*>(buf3 + L::TILE)[i] = u32x4{0u, 0u, 0u, 0u};
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  int id0 = load_id(0), id1 = load_id(1), id2 = load_id(2), id3;   // of tile j in id(j % 4)
+  load_tile(0, id0, buf0);
+  load_tile(1, id1, buf1);
+  // Q arrives here: waited for inside the loop, where the compiler cannot see
+  // the tile loads, it would drain them in every step
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    u32x4 w = __builtin_bit_cast(u32x4, qb[c]);
+    asm volatile("" : "+v"(w));
+    qb[c] = __builtin_bit_cast(vec8, w);
+  }
   auto step = [&](int t, unsigned char* cur, unsigned char* prev, unsigned char* nxt2,
-                  int* ids_t2, int* ids_t3) {
+                  int& id_t2, int& id_t3) {
     // Every tile load but the latest step's has landed; after the barrier,
     // every wave's have. (A fenced barrier would wait for all of them.)
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LPT) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LPT) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    load_tile(t + 2, ids_t2, nxt2);
+    load_tile(t + 2, id_t2, nxt2);
     compute(t, cur, prev + L::TILE);
     // (after the tile's LDS reads: a scalar load in flight would make every
     // wait for them a wait for it too)
-    load_ids(t + 3, ids_t3);
+    id_t3 = load_id(t + 3);
   };
   unsigned char* last = buf0;   // the buffer of the last tile computed
   for (int t = 0;; t += 4) {
-    step(t, buf0, buf3, buf2, ids2, ids3);
+    step(t, buf0, buf3, buf2, id2, id3);
     last = buf0;
     if (t + 1 >= ntiles) break;
-    step(t + 1, buf1, buf0, buf3, ids3, ids0);
+    step(t + 1, buf1, buf0, buf3, id3, id0);
     last = buf1;
     if (t + 2 >= ntiles) break;
-    step(t + 2, buf2, buf1, buf0, ids0, ids1);
+    step(t + 2, buf2, buf1, buf0, id0, id1);
     last = buf2;
     if (t + 3 >= ntiles) break;
-    step(t + 3, buf3, buf2, buf1, ids1, ids2);
+    step(t + 3, buf3, buf2, buf1, id1, id2);
     last = buf3;
     if (t + 4 >= ntiles) break;
   }
