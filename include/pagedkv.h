@@ -87,7 +87,9 @@ int pkv_append_kv(void* k_pool, void* v_pool, int64_t num_slots,
  * 27..30 and an out-of-range flag in bit 31), and n_items items {seq,
  * n_pages, first token, kv_len, partial slot (-1: a whole sequence), pieces
  * of the sequence, its first slot, flags (bit 0: the piece holds the
- * sequence's last page)} at the end of the block, item i at 8 (i + 1) ints
+ * sequence's last page; from bit 1: the sequence's row of q, out, k_new, v_new
+ * and slot_mapping, its index as planned -- a caller whose batch is part of
+ * a larger one may set it to a row of the larger one's arrays)} at the end of the block, item i at 8 (i + 1) ints
  * before the next block -- pieces of cut sequences before their last, whole
  * sequences, then the last pieces; then 64 zero ints. *plan_stride_out is at
  * least 68.

@@ -94,11 +94,16 @@ def _decode_ptrs(indptr, indices, kv_lens, plan, slots) -> tuple:
 
 class _DecodeRows:
     """The one-token sequences of a mixed batch, run through the decode kernel:
-    their token rows in q/out, and their paging metadata and decode plan as a
-    batch of their own."""
+    their decode plan as a batch of their own, whose items name their token
+    rows in the whole batch's q and out. The rest (rows, CSR, lengths) is on
+    the host until asked for: the decode kernel reads only the plan."""
 
-    __slots__ = ("rows", "indptr", "indices", "kv_lens", "plan", "n", "n_work", "n_slots",
-                 "stride")
+    __slots__ = ("plan", "n", "n_work", "n_slots", "stride", "_host", "_put")
+
+    rows = property(lambda self: self._put(self._host[0]))
+    indptr = property(lambda self: self._put(self._host[1]))
+    kv_lens = property(lambda self: self._put(self._host[2]))
+    indices = property(lambda self: self._put(self._host[3]))
 
 
 class _Pending:
@@ -459,12 +464,8 @@ class MI355XBackend:
             _native.check(rc, "attend (prefill)")
             d = p.dec
             if d is not None:
-                qd = q.index_select(0, d.rows)
-                od = torch.empty_like(qd)
-                self._launch_decode(qd, od, kp, vp, _decode_ptrs(d.indptr, d.indices,
-                                                                 d.kv_lens, d.plan, None),
-                                    d.n, d.n_work, d.n_slots, d.stride, scale, stream, None)
-                out.index_copy_(0, d.rows, od)
+                self._launch_decode(q, out, kp, vp, p.ptrs, d.n, d.n_work, d.n_slots, d.stride,
+                                    scale, stream, None)
         return out
 
     def _launch_decode(self, q, out, kp, vp, ptrs, n_seqs, n_work, n_slots, stride, scale,
@@ -545,7 +546,7 @@ class MI355XBackend:
                              f"for {p.n_tokens} tokens")
         i32 = lambda a: np.ascontiguousarray(a, dtype=np.int32)  # noqa: E731
         kvl32, indptr32, last32, cu32 = i32(kvl), i32(indptr), i32(last), i32(cu)
-        ptr = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+        ptr = lambda a: a.ctypes.data  # noqa: E731
         decodes = None
         p.stride = 0
         if not use_prefill:
@@ -570,12 +571,13 @@ class MI355XBackend:
         p.kv_lens = self._dev_i32(meta.kv_lens)
         p.dec = None
         if decodes is not None:
-            p.dec = self._decode_rows(decodes, cu, indptr, kvl, last, indices, p.indices)
+            p.dec = self._decode_rows(decodes, cu, indptr, kvl, last, indices)
         p.cu_q = self._dev_i32(meta.cu_query_lens)
         p.bidx = self._dev_i32(meta.batch_indices)
         p.slots = (self._dev_i32(meta.slot_mapping) if meta.slot_mapping is not None
                    else None)
-        p.ptrs = _decode_ptrs(p.indptr, p.indices, p.kv_lens, p.plan, p.slots)
+        p.ptrs = _decode_ptrs(p.indptr, p.indices, p.kv_lens,
+                              p.plan if p.dec is None else p.dec.plan, p.slots)
         self._planned = p
         self.n_plans += 1
         return p
@@ -585,7 +587,7 @@ class MI355XBackend:
         Returns (plan, n_work, n_slots, stride)."""
         if not self._fast_decode:  # the generic kernel reads the CSR, not a plan
             return np.zeros(4, dtype=np.int32), 1, 0, 4
-        ptr = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+        ptr = lambda a: a.ctypes.data  # noqa: E731
         n_work, n_slots, stride = C.c_int32(), C.c_int32(), C.c_int32()
         needed = C.c_int64()
         cap = 6 * self._decode_wgs + 2 * int(indptr32[-1]) + 24 * n + 128
@@ -627,23 +629,32 @@ class MI355XBackend:
         self._ws_zero = counter_bytes
         return (buf[:int(needed.value)].copy(), n_work.value, n_slots.value, stride.value)
 
-    def _decode_rows(self, dec, cu, indptr, kvl, last, indices, indices_dev) -> _DecodeRows:
+    def _decode_rows(self, dec, cu, indptr, kvl, last, indices) -> _DecodeRows:
         """The decode-kernel batch of a mixed batch's one-token sequences
-        ``dec``: their own CSR over a gathered copy of their page ids."""
+        ``dec``: a plan over their own pages, each item's row set to the
+        sequence's token row in the whole batch, so the kernel reads q and
+        writes out in place."""
         npg = indptr[dec + 1] - indptr[dec]
         sub_ptr = np.concatenate([[0], np.cumsum(npg)])
         # position in the batch's kv_indices of every page of the sub-batch
         page_ix = np.repeat(indptr[dec] - sub_ptr[:-1], npg) + np.arange(int(sub_ptr[-1]))
         i32 = lambda a: np.ascontiguousarray(a, dtype=np.int32)  # noqa: E731
+        rows = cu[dec]
+        host = (rows.astype(np.int64), i32(sub_ptr), i32(kvl[dec]), i32(indices[page_ix]))
         d = _DecodeRows()
         d.n = int(dec.shape[0])
-        plan, d.n_work, d.n_slots, d.stride = self._plan_decode(
-            i32(sub_ptr), i32(indices[page_ix]), i32(kvl[dec]), i32(last[dec]), d.n)
+        plan, d.n_work, d.n_slots, d.stride = self._plan_decode(host[1], host[3], host[2],
+                                                                i32(last[dec]), d.n)
+        # item i of a bin: 8 (i + 1) ints before the bin's end; its sequence
+        # first, its flags (last-page bit, then the row) last
+        blocks = plan[:plan.shape[0] // d.stride * d.stride].reshape(-1, d.stride)
+        count = blocks[:, 0]
+        bins = np.repeat(np.arange(blocks.shape[0]), count)
+        first = np.repeat(np.cumsum(count) - count, count)
+        at = (bins + 1) * d.stride - 8 * (np.arange(bins.shape[0]) - first + 1)
+        plan[at + 7] = (plan[at + 7] & 1) | (rows[plan[at]] << 1)
         d.plan = self._upload(plan)
-        d.rows = self._upload(cu[dec].astype(np.int64))
-        d.indptr = self._upload(i32(sub_ptr))
-        d.kv_lens = self._upload(i32(kvl[dec]))
-        d.indices = indices_dev.index_select(0, self._upload(page_ix.astype(np.int64)))
+        d._host, d._put = host, self._upload
         return d
 
     def _upload(self, a: np.ndarray) -> torch.Tensor:

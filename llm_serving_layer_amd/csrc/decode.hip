@@ -88,6 +88,9 @@ constexpr int kHdrInts = 4;         // bin header {n_items, n_pages, 0, 0}
 constexpr int kItemInts = 8;        // {seq, n_pages, first token, kv_len, slot, n_pieces,
                                     //  first slot, flags}
 constexpr int kItemLast = 1;        // flags: the piece holds its sequence's last page
+constexpr int kRowShift = 1;        // flags: the sequence's row of q, out, k_new, v_new and
+                                    // slot_mapping from this bit on (its index, unless the
+                                    // batch is part of a larger one)
 constexpr int kStageMax = 8;        // items staged in LDS at a time (at most)
 constexpr int kPlanTail = 64;       // zero ints after the last bin (words read past its end)
 constexpr int kMinTail = 4;         // a remainder of a cut below this (and below half a
@@ -106,7 +109,7 @@ template <int D, int G> struct PartLayout {
   static constexpr int FLOATS = NGR * NDB * 64;  // per (slot, KV head)
 };
 
-// Split-K merge for one KV head h of sequence seq, run by the wave that
+// Split-K merge for one KV head h of a sequence (row orow of out), run by the wave that
 // published the last partial, or by the sequence's last piece with its own
 // partial still in registers (`own`). Lanes run over partitions for each
 // head row's max M and sum L; then, 64 partitions at a time, the weights
@@ -122,7 +125,7 @@ template <int D, int G> struct PartLayout {
 // the result does not depend on the batch or on which wave merges.
 // NBW dim blocks from b0 on are merged (all of them by default).
 template <typename T, int D, int G, int NBW = D / 16>
-__device__ __forceinline__ void merge_head(T* __restrict__ out, float* wts, int seq, int h,
+__device__ __forceinline__ void merge_head(T* __restrict__ out, float* wts, int orow, int h,
                                            int n_kv_heads, int nparts, int slot0,
                                            __amdgpu_buffer_rsrc_t ro, __amdgpu_buffer_rsrc_t rm,
                                            bool own, const f32x4* own_o, float own_m,
@@ -223,7 +226,7 @@ __device__ __forceinline__ void merge_head(T* __restrict__ out, float* wts, int 
         const float inv = 1.f / lr_;   // one division per row, not per element
 #pragma unroll
         for (int b = 0; b < NBW; ++b)
-          out[((int64_t)seq * Hq + h * G + r) * D + 16 * (b0 + b) + n] = (T)(acc[b][i] * inv);
+          out[((int64_t)orow * Hq + h * G + r) * D + 16 * (b0 + b) + n] = (T)(acc[b][i] * inv);
       }
     }
   }
@@ -359,14 +362,11 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
   const int32_t* items_end = bp + stride;   // item i: items_end - (i + 1) * kItemInts
   typedef Stage<T, D, G> SG;
   static_assert(SG::C <= kStageMax, "the first batch's items lie inside the block");
-  // read together with the header: the first batch's (seq, flags), the
-  // first item and the first two page words
-  int sq0[SG::C], fl0[SG::C];
+  // read together with the header: the first batch's flags, the first item and
+  // the first two page words
+  int fl0[SG::C];
 #pragma unroll
-  for (int j = 0; j < SG::C; ++j) {
-    sq0[j] = items_end[-(j + 1) * kItemInts];
-    fl0[j] = items_end[-(j + 1) * kItemInts + 7];
-  }
+  for (int j = 0; j < SG::C; ++j) fl0[j] = items_end[-(j + 1) * kItemInts + 7];
   struct Item { int seq, np, tok0, kv, slot, nparts, slot0, flags; };
   auto item_at = [&](int i) __attribute__((always_inline)) -> Item {
     const int32_t* it = items_end - (int64_t)(i + 1) * kItemInts;
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
   // (keeps every one of these reads ahead of the branch below, so they go
   // out together instead of after it)
 #pragma unroll
-  for (int j = 0; j < SG::C; ++j) asm volatile("" ::"s"(sq0[j]), "s"(fl0[j]));
+  for (int j = 0; j < SG::C; ++j) asm volatile("" ::"s"(fl0[j]));
   asm volatile("" ::"s"(cur.seq), "s"(cur.np), "s"(cur.tok0), "s"(cur.kv), "s"(cur.slot),
                "s"(cur.nparts), "s"(cur.slot0), "s"(cur.flags), "s"(wcur), "s"(wnext), "s"(q),
                "s"(k_new), "s"(v_new));
@@ -417,39 +417,32 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
   // Loads of the slots of items i0 .. i0 + C - 1: lane chunk c = 64 r + lane
   // is 16 bytes w of item i's slot (Q rows of the KV head's G query heads,
   // then the KV head's slice of the new K row and of the new V row).
-  // (seq, flags) of items i0 .. i0 + C - 1 (the last item repeated past the end)
-  auto stage_fields = [&](int i0, int* sq, int* fl) __attribute__((always_inline)) {
+  // flags of items i0 .. i0 + C - 1 (the last item repeated past the end)
+  auto stage_fields = [&](int i0, int* fl) __attribute__((always_inline)) {
     const int ns = min(SG::C, n_items - i0);
 #pragma unroll
-    for (int j = 0; j < SG::C; ++j) {
-      const int32_t* it = items_end - (int64_t)(i0 + min(j, ns - 1) + 1) * kItemInts;
-      sq[j] = it[0];
-      fl[j] = it[7];
-    }
+    for (int j = 0; j < SG::C; ++j)
+      fl[j] = (items_end - (int64_t)(i0 + min(j, ns - 1) + 1) * kItemInts)[7];
   };
-  auto stage_load = [&](int i0, const int* sq, const int* fl, u32x4* d)
-                        __attribute__((always_inline)) {
+  auto stage_load = [&](int i0, const int* fl, u32x4* d) __attribute__((always_inline)) {
     const int ns = min(SG::C, n_items - i0);
 #pragma unroll
     for (int r = 0; r < SG::ROUNDS; ++r) {
       const int c = r * 64 + lane;
       const int i = c / SG::CPI, w = c - i * SG::CPI;
-      // item i's fields by masks (a select chain here becomes a lookup
+      // item i's flags by masks (a select chain here becomes a lookup
       // table in scratch memory)
-      int si = 0, fi = 0;
+      int fi = 0;
 #pragma unroll
-      for (int j = 0; j < SG::C; ++j) {
-        const int msk = -(int)(i == j);
-        si |= sq[j] & msk;
-        fi |= fl[j] & msk;
-      }
+      for (int j = 0; j < SG::C; ++j) fi |= fl[j] & -(int)(i == j);
+      const int64_t ri = fi >> kRowShift;
       const unsigned char* src = nullptr;
       if (i < ns) {
         if (w < SG::QC)
-          src = reinterpret_cast<const unsigned char*>(q + ((int64_t)si * Hq + h * G) * D) + w * 16;
+          src = reinterpret_cast<const unsigned char*>(q + (ri * Hq + h * G) * D) + w * 16;
         else if (fuse && (fi & kItemLast))
           src = reinterpret_cast<const unsigned char*>(
-                    (w < SG::QC + SG::RC ? k_new : v_new) + (int64_t)si * row_elems + h * D) +
+                    (w < SG::QC + SG::RC ? k_new : v_new) + ri * row_elems + h * D) +
                 (w < SG::QC + SG::RC ? w - SG::QC : w - SG::QC - SG::RC) * 16;
       }
       // each read once per item: streaming hint
@@ -466,7 +459,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
     wave_lds_sync();
   };
   u32x4 sgd[SG::ROUNDS];
-  stage_load(0, sq0, fl0, sgd);
+  stage_load(0, fl0, sgd);
   // One page in flight: its registers and its word; the next page's word is
   // read a step ahead.
   vec8 kr[NLD], vr[NLD];
@@ -488,7 +481,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
     }
     kx = *reinterpret_cast<const vec8*>(sl + SG::QB + lcol);
     vx = *reinterpret_cast<const vec8*>(sl + SG::QB + RB + lcol);
-    new_slot = (fuse && (cur.flags & kItemLast)) ? slot_mapping[cur.seq] : 0;
+    new_slot = (fuse && (cur.flags & kItemLast)) ? slot_mapping[cur.flags >> kRowShift] : 0;
   };
   take_item(0);
   int it_idx = 0;
@@ -631,9 +624,9 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
   };
 
   // Merge (seq, h) from the stored partials and reset its counter.
-  auto merge = [&](int sq, int nparts, int slot0, bool own) __attribute__((always_inline)) {
+  auto merge = [&](int sq, int orow, int nparts, int slot0, bool own) __attribute__((always_inline)) {
     PKV_TL(const unsigned long long tm = __builtin_amdgcn_s_memrealtime(); ++tl_merges;)
-    merge_head<T, D, G>(out, reinterpret_cast<float*>(kl), sq, h, n_kv_heads, nparts, slot0,
+    merge_head<T, D, G>(out, reinterpret_cast<float*>(kl), orow, h, n_kv_heads, nparts, slot0,
                         ro, rm, own, o, m_run, l_run);
     if (lane == 0)
       __hip_atomic_store(counters + (int64_t)sq * n_kv_heads + h, 0, __ATOMIC_RELAXED,
@@ -650,11 +643,11 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
   };
   // A deferred arrival: pa_state 1 once a partial is stored; it is counted
   // at page pa_at.
-  int pa_state = 0, pa_at = 0, pa_seq = 0, pa_nparts = 0, pa_slot0 = 0, pa_old = 0;
+  int pa_state = 0, pa_at = 0, pa_seq = 0, pa_row = 0, pa_nparts = 0, pa_slot0 = 0, pa_old = 0;
   // check a counted arrival: the last one merges
   auto finish_arrival = [&]() __attribute__((always_inline)) {
     if (__builtin_amdgcn_readfirstlane(pa_old) == pa_nparts - 1)
-      merge(pa_seq, pa_nparts, pa_slot0, false);
+      merge(pa_seq, pa_row, pa_nparts, pa_slot0, false);
     pa_state = 0;
   };
   auto flush_arrival = [&]() __attribute__((always_inline)) {  // count a pending arrival now
@@ -670,7 +663,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
   auto end_item = [&](int p) __attribute__((always_inline)) {
     if (cur.slot < 0) {
       finish_out();
-      if (lane == 0) ring_seq[n_out] = cur.seq;
+      if (lane == 0) ring_seq[n_out] = cur.flags >> kRowShift;
       ring_full = ++n_out == RG::KO;
     } else {
       flush_arrival();   // at most one deferred arrival at a time
@@ -679,7 +672,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
         // the sequence's last piece, and every other piece had arrived when
         // it started: it merges, its own partial straight from registers,
         // and publishes nothing
-        merge(cur.seq, cur.nparts, cur.slot0, true);
+        merge(cur.seq, cur.flags >> kRowShift, cur.nparts, cur.slot0, true);
       } else {
         const uint32_t head_off =
             (uint32_t)(((int64_t)cur.slot * n_kv_heads + h) * PL::FLOATS * 4);
@@ -696,6 +689,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
               (uint32_t)(((int64_t)cur.slot * Hq + h * G + lane) * 8), 0, kSc1);
         asm volatile("" ::: "memory");  // the stores stay before the loads that follow
         pa_seq = cur.seq;
+        pa_row = cur.flags >> kRowShift;
         pa_nparts = cur.nparts;
         pa_slot0 = cur.slot0;
         if (!last && p + 2 < n_pages) {
@@ -714,9 +708,9 @@ __global__ __launch_bounds__(kMaxWaves * 64) void decode_kernel(
     ++it_idx;
     if (it_idx < n_items) {
       if (it_idx % SG::C == 0) {   // the next batch of slots
-        int sq[SG::C], fl[SG::C];
-        stage_fields(it_idx, sq, fl);
-        stage_load(it_idx, sq, fl, sgd);
+        int fl[SG::C];
+        stage_fields(it_idx, fl);
+        stage_load(it_idx, fl, sgd);
         stage_store(sgd);
       }
       cur = nxt;
@@ -926,6 +920,7 @@ __global__ __launch_bounds__(256) void decode_piece_kernel(
     const int32_t* it = bp + stride - (int64_t)(item + 1) * kItemInts;
     const int seq = it[0], np = it[1], tok0 = it[2], kv = it[3], slot = it[4], nparts = it[5],
               slot0 = it[6];
+    const int row = it[7] >> kRowShift;
     const bool fuse = k_new != nullptr && (it[7] & kItemLast);
     // the first chunk's page words, word i in lane i (reads past the bin's
     // words stay inside the plan: kPlanTail)
@@ -938,18 +933,18 @@ __global__ __launch_bounds__(256) void decode_piece_kernel(
       qb[c] = vec8{};
       kx[c] = vec8{};
       if (n < G)
-        qb[c] = *reinterpret_cast<const vec8*>(q + ((int64_t)seq * Hq + h * G + n) * D + c * 32 +
+        qb[c] = *reinterpret_cast<const vec8*>(q + ((int64_t)row * Hq + h * G + n) * D + c * 32 +
                                                g * 8);
     }
     // the new row: K as the QK A operand has it, V in 16-byte chunks
     int new_slot = 0;
     if (fuse) {
-      const int64_t at = (int64_t)seq * row_elems + h * D;
+      const int64_t at = (int64_t)row * row_elems + h * D;
 #pragma unroll
       for (int c = 0; c < NCH; ++c)
         kx[c] = *reinterpret_cast<const vec8*>(k_new + at + c * 32 + g * 8);
       vx = *reinterpret_cast<const vec8*>(v_new + at + lc * 8);
-      new_slot = slot_mapping[seq];
+      new_slot = slot_mapping[row];
     }
 
     f32x4 o[NBW];
@@ -1163,7 +1158,7 @@ __global__ __launch_bounds__(256) void decode_piece_kernel(
           const float inv = 1.f / li;
 #pragma unroll
           for (int b = 0; b < NBW; ++b)
-            out[((int64_t)seq * Hq + h * G + r) * D + 16 * (wave * NBW + b) + n] =
+            out[((int64_t)row * Hq + h * G + r) * D + 16 * (wave * NBW + b) + n] =
                 (T)(o[b][e] * inv);
         }
       }
@@ -1188,7 +1183,7 @@ __global__ __launch_bounds__(256) void decode_piece_kernel(
         *arrived = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
       if (*arrived == nparts - 1) {
-        merge_head<T, D, G, NBW>(out, reinterpret_cast<float*>(vt) + wave * 64 * 4 * NGR, seq, h,
+        merge_head<T, D, G, NBW>(out, reinterpret_cast<float*>(vt) + wave * 64 * 4 * NGR, row, h,
                                  n_kv_heads, nparts, slot0, ro, rm, false, o, m_run, l_run,
                                  wave * NBW);
         if (threadIdx.x == 0)
@@ -1441,7 +1436,8 @@ extern "C" int pkv_plan_decode(const int32_t* kv_indptr, const int32_t* kv_indic
       }
       const bool last = x.first + x.np == np_seq;
       const int32_t vals[kItemInts] = {x.seq, x.np, x.first * page_size, kv_lens[x.seq],
-                                       x.slot, x.nparts, x.slot0, last ? kItemLast : 0};
+                                       x.slot, x.nparts, x.slot0,
+                                       (x.seq << kRowShift) | (last ? kItemLast : 0)};
       for (int k = 0; k < kItemInts; ++k) *it++ = vals[k];
     }
   }

@@ -16,7 +16,7 @@ import torch
 from llm_serving_layer_amd import BlockAllocator, SequenceBlocks
 from llm_serving_layer_amd.backend import MI355XBackend
 
-from ._util import grow_and_assemble
+from ._util import grow_and_assemble, make_meta
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -70,3 +70,28 @@ def test_small_and_large_batches_give_the_same_bits(n_heads, d, dtype, part_page
     assert torch.equal(few.v_pool[0].view(torch.int16), big.v_pool[0].view(torch.int16))
     big.check_device_errors()
     few.check_device_errors()
+
+
+@pytest.mark.parametrize("n_decode", [3, 300])
+def test_decodes_of_a_mixed_batch_read_and_write_their_token_rows(n_decode):
+    """Decodes between prompt chunks (rows 7, 8, ... of q and out, then past a
+    second chunk): either kernel gives them the bits they have alone."""
+    print(f"mixed rows n_decode={n_decode}", flush=True)
+    lens = [0] + (EDGES * 12)[1:n_decode + 1] + [33]
+    counts = [7] + [1] * n_decode + [20]
+    alloc = BlockAllocator(8192, 16)
+    seqs = [SequenceBlocks(alloc, seq_id=i) for i in range(len(lens))]
+    for s, n in zip(seqs, lens):
+        if n:
+            s.append(n)
+    bk = MI355XBackend(1, 8192, 16, 1, 4, 64, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(4)
+    bk.k_pool[0].normal_(generator=g)
+    bk.v_pool[0].normal_(generator=g)
+    q = torch.randn(sum(counts), 4, 64, generator=g, device=DEV).half()
+    meta = grow_and_assemble(seqs, counts, 16, device=DEV)
+    out = bk.attend(q, 0, 0.125, meta)
+    assert (bk._planned.dec.n_work >= 256) == (n_decode == 300)
+    alone = make_meta(seqs[1:-1], [1] * n_decode, 16, device=DEV)
+    assert torch.equal(bk.attend(q[7:7 + n_decode], 0, 0.125, alone), out[7:7 + n_decode])
+    bk.check_device_errors()
