@@ -244,6 +244,25 @@ int pkv_attend_prefill(const void* q, void* out,
                        int32_t* status_word, void* stream);
 
 /*
+ * pkv_attend_prefill over the chunks of a mixed batch and pkv_attend_decode
+ * over its one-token sequences, with the same result as the two calls: one
+ * launch where neither fills the chip. prefill_plan covers the multi-token
+ * sequences only; decode_plan is pkv_plan_decode's output over the n_decodes
+ * one-token sequences, its items' rows set to their token rows of q and out.
+ * No reference counterpart: the reference attends a mixed batch sequence by
+ * sequence (serving/backends/paged_torch.py:280-485).
+ */
+int pkv_attend_mixed(const void* q, void* out, void* k_pool, void* v_pool, int64_t num_blocks,
+                     const int32_t* cu_query_lens, const int32_t* kv_indptr,
+                     const int32_t* kv_indices, const int32_t* kv_lens,
+                     const int32_t* batch_indices, int32_t n_seqs, int32_t n_tokens,
+                     int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int32_t page_size,
+                     float scale, int32_t dtype, const int32_t* prefill_plan, int32_t n_tiles,
+                     int32_t q_tile, const int32_t* decode_plan, int32_t n_decodes,
+                     int32_t n_work, int32_t n_slots, int32_t plan_stride, void* workspace,
+                     int64_t workspace_bytes, int32_t* status_word, void* stream);
+
+/*
  * Batched block copy over every layer, K and V — replaces
  * PagedTorchBackend.copy_block (serving/backends/paged_torch.py:181-207),
  * called once per pair by RadixCache.ensure_writable

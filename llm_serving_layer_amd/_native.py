@@ -15,7 +15,7 @@ from pathlib import Path
 # PKV_LIBRARY selects another build of the same library (e.g. a tuning variant).
 LIB_PATH = Path(os.environ.get("PKV_LIBRARY") or
                 Path(__file__).resolve().parent / "_native" / "libpagedkv.so")
-ABI_VERSION = 11
+ABI_VERSION = 12
 
 DTYPE_F16, DTYPE_BF16, DTYPE_F32 = 0, 1, 2
 DECODE_SCRATCH_BYTES = 64 * 1024 * 1024   # PKV_DECODE_SCRATCH_BYTES
@@ -45,6 +45,9 @@ SIGNATURES = {
     "pkv_attend_prefill": (C.c_int, [_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _i32, _i32,
                                      _i32, _i32, _i32, _i32, _f32, _i32, _p, _i32, _i32, _p,
                                      _p]),
+    "pkv_attend_mixed": (C.c_int, [_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _i32, _i32, _i32,
+                                   _i32, _i32, _i32, _f32, _i32, _p, _i32, _i32, _p, _i32, _i32,
+                                   _i32, _i32, _p, _i64, _p, _p]),
     "pkv_copy_blocks": (C.c_int, [_p, _i32, _i64, _i64, _i64, _p, _p, _i32, _p, _p]),
     "pkv_gather_blocks": (C.c_int, [_p, _i32, _i64, _i64, _i64, _p, _i32, _p, _p, _p]),
     "pkv_scatter_blocks": (C.c_int, [_p, _i32, _i64, _i64, _i64, _p, _i32, _p, _p, _p]),

@@ -83,7 +83,7 @@ class _Plan:
 
     __slots__ = ("meta", "use_prefill", "slots", "indptr", "indices", "kv_lens", "cu_q",
                  "bidx", "plan", "n_work", "n_slots", "stride", "n_tokens", "n_seqs", "fusable",
-                 "dec", "ptrs")
+                 "dec", "ptrs", "pre_ptrs")
 
 
 def _decode_ptrs(indptr, indices, kv_lens, plan, slots) -> tuple:
@@ -98,7 +98,7 @@ class _DecodeRows:
     rows in the whole batch's q and out. The rest (rows, CSR, lengths) is on
     the host until asked for: the decode kernel reads only the plan."""
 
-    __slots__ = ("plan", "n", "n_work", "n_slots", "stride", "_host", "_put")
+    __slots__ = ("plan", "ptr", "n", "n_work", "n_slots", "stride", "_host", "_put")
 
     rows = property(lambda self: self._put(self._host[0]))
     indptr = property(lambda self: self._put(self._host[1]))
@@ -455,17 +455,19 @@ class MI355XBackend:
             self._launch_decode(q, out, kp, vp, p.ptrs, p.n_seqs, p.n_work, p.n_slots,
                                 p.stride, scale, stream, pend if fused else None)
         else:
-            rc = self._lib.pkv_attend_prefill(
-                q.data_ptr(), out.data_ptr(), kp, vp, self.num_blocks, p.cu_q.data_ptr(),
-                p.indptr.data_ptr(), p.indices.data_ptr(), p.kv_lens.data_ptr(),
-                p.bidx.data_ptr(), p.n_seqs, p.n_tokens, self.n_heads, self.n_kv_heads,
-                self.head_dim, self.block_size, float(scale), self._code, p.plan.data_ptr(),
-                p.n_work, self.q_tile, self._status.data_ptr(), stream)
-            _native.check(rc, "attend (prefill)")
+            cu_q, indptr, indices, kv_lens, bidx, plan = p.pre_ptrs
+            batch = (q.data_ptr(), out.data_ptr(), kp, vp, self.num_blocks, cu_q, indptr, indices,
+                     kv_lens, bidx, p.n_seqs, p.n_tokens, self.n_heads, self.n_kv_heads,
+                     self.head_dim, self.block_size, float(scale), self._code, plan, p.n_work,
+                     self.q_tile)
             d = p.dec
-            if d is not None:
-                self._launch_decode(q, out, kp, vp, p.ptrs, d.n, d.n_work, d.n_slots, d.stride,
-                                    scale, stream, None)
+            if d is None:
+                rc = self._lib.pkv_attend_prefill(*batch, self._status_ptr, stream)
+            else:
+                rc = self._lib.pkv_attend_mixed(*batch, d.ptr, d.n, d.n_work, d.n_slots, d.stride,
+                                                self._ws_ptr, self._ws_bytes, self._status_ptr,
+                                                stream)
+            _native.check(rc, "attend (prefill)")
         return out
 
     def _launch_decode(self, q, out, kp, vp, ptrs, n_seqs, n_work, n_slots, stride, scale,
@@ -576,8 +578,9 @@ class MI355XBackend:
         p.bidx = self._dev_i32(meta.batch_indices)
         p.slots = (self._dev_i32(meta.slot_mapping) if meta.slot_mapping is not None
                    else None)
-        p.ptrs = _decode_ptrs(p.indptr, p.indices, p.kv_lens,
-                              p.plan if p.dec is None else p.dec.plan, p.slots)
+        p.ptrs = _decode_ptrs(p.indptr, p.indices, p.kv_lens, p.plan, p.slots)
+        p.pre_ptrs = tuple(t.data_ptr() for t in (p.cu_q, p.indptr, p.indices, p.kv_lens, p.bidx,
+                                                  p.plan))
         self._planned = p
         self.n_plans += 1
         return p
@@ -654,6 +657,7 @@ class MI355XBackend:
         at = (bins + 1) * d.stride - 8 * (np.arange(bins.shape[0]) - first + 1)
         plan[at + 7] = (plan[at + 7] & 1) | (rows[plan[at]] << 1)
         d.plan = self._upload(plan)
+        d.ptr = d.plan.data_ptr()
         d._host, d._put = host, self._upload
         return d
 

@@ -196,7 +196,7 @@ int pkv_upload_pinned(void* dst, const void* host, int64_t bytes, void* stream) 
   return PKV_OK;
 }
 
-int pkv_abi_version(void) { return 11; }
+int pkv_abi_version(void) { return 12; }
 
 const char* pkv_last_error(void) { return g_err.c_str(); }
 
