@@ -225,13 +225,15 @@ __device__ __forceinline__ void decode_piece(
 
   const int32_t* bp = plan + (int64_t)bin * stride;
   const int32_t* words = bp + kHdrInts;
-  const int n_items = bp[0];
   const __amdgpu_buffer_rsrc_t ro = ws_rsrc(part_o, o_bytes);
   const __amdgpu_buffer_rsrc_t rm = ws_rsrc(part_ml, ml_bytes);
 
-  // (one item, unless the plan was made for fewer workgroups than fit)
+  // One item, unless the plan was made for fewer workgroups than fit. (The
+  // count, the item and its words come in one round trip; the slot below a
+  // bin's last item still lies inside its plan block.)
+  const int n_items = bp[0];
   int p0 = 0;
-  for (int item = 0; item < n_items; ++item) {
+  for (int item = 0;; ++item) {
     const int32_t* it = bp + stride - (int64_t)(item + 1) * kItemInts;
     const int seq = it[0], np = it[1], tok0 = it[2], kv = it[3], slot = it[4], nparts = it[5],
               slot0 = it[6];
@@ -240,6 +242,8 @@ __device__ __forceinline__ void decode_piece(
     // the first chunk's page words, word i in lane i (reads past the bin's
     // words stay inside the plan: kPlanTail)
     int wd = words[p0 + lane];
+    asm volatile("" ::"s"(seq), "s"(np), "s"(kv), "s"(it[7]), "s"(n_items));
+    if (item >= n_items) break;
 
     // Q^T, the QK B operand (column n = query head h*G + n, zero beyond G)
     vec8 qb[NCH], kx[NCH], vx{};
@@ -314,20 +318,14 @@ __device__ __forceinline__ void decode_piece(
       const bool tail = c0 + cn == np;
       const int jt = cn - 1;
       const uint32_t wt = (uint32_t)__builtin_amdgcn_readlane(wd, jt);
-      bool patch = false;
+      bool patch = false, store = false;
       const int tl = (kv - 1) % PS;
       if (fuse && tail && wave == (jt & 3)) {
         if (new_slot < 0 || (int64_t)new_slot >= num_blocks * PS) {
           if (lane == 0) flag(status, PKV_STATUS_BAD_SLOT);
         } else {
           patch = (int64_t)new_slot == (int64_t)(wt & ((1u << kPageIdBits) - 1)) * PS + tl;
-          const int64_t dst = (int64_t)new_slot * row_elems + h * D;
-          if (n == 0) {
-#pragma unroll
-            for (int c = 0; c < NCH; ++c)
-              *reinterpret_cast<vec8*>(kpool + dst + c * 32 + g * 8) = kx[c];
-          }
-          if (lane < CPR) *reinterpret_cast<vec8*>(vpool + dst + lc * 8) = vx;
+          store = true;
 #pragma unroll
           for (int i = 0; i < PW; ++i) {
             if (patch && 4 * i + wave == jt && n == tl) {
@@ -374,6 +372,15 @@ __device__ __forceinline__ void decode_piece(
         }
       }
       __syncthreads();
+      if (store) {   // (here, so that the wait for V is not a wait for it)
+        const int64_t dst = (int64_t)new_slot * row_elems + h * D;
+        if (n == 0) {
+#pragma unroll
+          for (int c = 0; c < NCH; ++c)
+            *reinterpret_cast<vec8*>(kpool + dst + c * 32 + g * 8) = kx[c];
+        }
+        if (lane < CPR) *reinterpret_cast<vec8*>(vpool + dst + lc * 8) = vx;
+      }
 
       // The running reference over the chunk's pages: it moves at a page when
       // some head's maximum is more than 8 above it. mv: bit j set where it
@@ -433,29 +440,51 @@ __device__ __forceinline__ void decode_piece(
 #pragma unroll
         for (int e = 0; e < 4; ++e) lsum[j + e] = t[e];
       }
+      auto move = [&](int j) __attribute__((always_inline)) {
+        const float m_new = fmaxf(m_run, mx[j]);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        l_run *= alpha;
+        m_run = m_new;
 #pragma unroll
-      for (int j = 0; j < CH; ++j) {
-        if (j < cn) {
-          if (mv >> j & 1) {
-            const float m_new = fmaxf(m_run, mx[j]);
-            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-            l_run *= alpha;
-            m_run = m_new;
+        for (int e = 0; e < 4; ++e) {
+          const float a = from_lane(alpha, e);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float a = from_lane(alpha, e);
+          for (int b = 0; b < NBW; ++b) o[b][e] *= a;
+        }
+      };
+      auto read_page = [&](int j, vec4& pr, vec4* v) __attribute__((always_inline)) {
+        pr = *reinterpret_cast<const vec4*>(pt + j * 512 + lane * 8);
 #pragma unroll
-              for (int b = 0; b < NBW; ++b) o[b][e] *= a;
+        for (int b = 0; b < NBW; ++b)
+          v[b] = __builtin_bit_cast(
+              vec4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(
+                        vt + j * L::VPAGE +
+                        swz<RB>(4 * g + (n >> 2), 16 * (wave * NBW + b) + 4 * (n & 3)))));
+      };
+      auto add_page = [&](int j, const vec4& pr, const vec4* v) __attribute__((always_inline)) {
+        l_run += lsum[j];
+#pragma unroll
+        for (int b = 0; b < NBW; ++b) o[b] = Mma<T>::pv(pr, v[b], o[b]);
+      };
+      if (mv & 1) move(0);
+      const bool moves = mv > 1;
+#pragma unroll
+      for (int j0 = 0; j0 < CH; j0 += 4) {
+        if (!moves && j0 + 4 <= cn) {   // four pages' reads at once
+          vec4 pr[4], v[4][NBW];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) read_page(j0 + j, pr[j], v[j]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) add_page(j0 + j, pr[j], v[j]);
+        } else {
+#pragma unroll
+          for (int j = j0; j < j0 + 4; ++j) {
+            if (j < cn) {
+              vec4 pr, v[NBW];
+              read_page(j, pr, v);
+              if (j > 0 && (mv >> j & 1)) move(j);
+              add_page(j, pr, v);
             }
-          }
-          l_run += lsum[j];
-          const vec4 pr = *reinterpret_cast<const vec4*>(pt + j * 512 + lane * 8);
-#pragma unroll
-          for (int b = 0; b < NBW; ++b) {
-            const i16x4 raw = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(
-                vt + j * L::VPAGE +
-                swz<RB>(4 * g + (n >> 2), 16 * (wave * NBW + b) + 4 * (n & 3))));
-            o[b] = Mma<T>::pv(pr, __builtin_bit_cast(vec4, raw), o[b]);
           }
         }
       }
