@@ -263,6 +263,36 @@ int pkv_attend_mixed(const void* q, void* out, void* k_pool, void* v_pool, int64
                      int64_t workspace_bytes, int32_t* status_word, void* stream);
 
 /*
+ * A batch's arguments that do not change from layer to layer, set once per
+ * step, and the two calls of a layer that read them: the same work as
+ * pkv_append_kv of the batch's n_tokens rows, and as pkv_attend_decode
+ * (is_prefill 0; k_new and v_new may be NULL), pkv_attend_prefill (n_decodes 0)
+ * or pkv_attend_mixed, at a third of the arguments a launch. The struct is
+ * read on the host before the call returns. No reference counterpart.
+ */
+typedef struct pkv_batch {
+  int64_t num_blocks;
+  const int32_t* cu_query_lens;
+  const int32_t* kv_indptr;
+  const int32_t* kv_indices;
+  const int32_t* kv_lens;
+  const int32_t* batch_indices;
+  const int32_t* slot_mapping;
+  const int32_t* prefill_plan;
+  const int32_t* decode_plan;
+  void* workspace;
+  int64_t workspace_bytes;
+  int32_t* status_word;
+  int32_t n_seqs, n_tokens, n_heads, n_kv_heads, head_dim, page_size, dtype, is_prefill;
+  int32_t n_tiles, q_tile, n_decodes, n_work, n_slots, plan_stride;
+} pkv_batch;
+
+int pkv_append_batch(const void* batch, void* k_pool, void* v_pool, const void* k,
+                     const void* v, void* stream);
+int pkv_attend_batch(const void* batch, const void* q, void* out, void* k_pool, void* v_pool,
+                     float scale, const void* k_new, const void* v_new, void* stream);
+
+/*
  * Batched block copy over every layer, K and V — replaces
  * PagedTorchBackend.copy_block (serving/backends/paged_torch.py:181-207),
  * called once per pair by RadixCache.ensure_writable

@@ -48,12 +48,27 @@ SIGNATURES = {
     "pkv_attend_mixed": (C.c_int, [_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _i32, _i32, _i32,
                                    _i32, _i32, _i32, _f32, _i32, _p, _i32, _i32, _p, _i32, _i32,
                                    _i32, _i32, _p, _i64, _p, _p]),
+    "pkv_append_batch": (C.c_int, [_p, _p, _p, _p, _p, _p]),
+    "pkv_attend_batch": (C.c_int, [_p, _p, _p, _p, _p, _f32, _p, _p, _p]),
     "pkv_copy_blocks": (C.c_int, [_p, _i32, _i64, _i64, _i64, _p, _p, _i32, _p, _p]),
     "pkv_gather_blocks": (C.c_int, [_p, _i32, _i64, _i64, _i64, _p, _i32, _p, _p, _p]),
     "pkv_scatter_blocks": (C.c_int, [_p, _i32, _i64, _i64, _i64, _p, _i32, _p, _p, _p]),
     "pkv_argmax_rows": (C.c_int, [_p, _i64, _i64, _i64, _i32, _p, _p]),
     "pkv_upload_pinned": (C.c_int, [_p, _p, _i64, _p]),
 }
+
+
+class Batch(C.Structure):
+    """``pkv_batch``: a batch's launch arguments, set once per plan."""
+
+    _fields_ = [("num_blocks", _i64), *[(n, _p) for n in (
+        "cu_query_lens", "kv_indptr", "kv_indices", "kv_lens", "batch_indices", "slot_mapping",
+        "prefill_plan", "decode_plan", "workspace")], ("workspace_bytes", _i64),
+        ("status_word", _p), *[(n, _i32) for n in (
+            "n_seqs", "n_tokens", "n_heads", "n_kv_heads", "head_dim", "page_size", "dtype",
+            "is_prefill", "n_tiles", "q_tile", "n_decodes", "n_work", "n_slots",
+            "plan_stride")]]
+
 
 _LIB = None
 _REASON = None

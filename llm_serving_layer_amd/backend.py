@@ -100,13 +100,7 @@ class _Plan:
 
     __slots__ = ("meta", "use_prefill", "slots", "indptr", "indices", "kv_lens", "cu_q",
                  "bidx", "plan", "n_work", "n_slots", "stride", "n_tokens", "n_seqs", "fusable",
-                 "dec", "ptrs", "pre_ptrs")
-
-
-def _decode_ptrs(indptr, indices, kv_lens, plan, slots) -> tuple:
-    """Device addresses a decode launch passes, taken once per plan."""
-    return (indptr.data_ptr(), indices.data_ptr(), kv_lens.data_ptr(), plan.data_ptr(),
-            slots.data_ptr() if slots is not None else None)
+                 "dec", "batch", "batch_ptr")
 
 
 class _DecodeRows:
@@ -115,7 +109,7 @@ class _DecodeRows:
     rows in the whole batch's q and out. The rest (rows, CSR, lengths) is on
     the host until asked for: the decode kernel reads only the plan."""
 
-    __slots__ = ("plan", "ptr", "n", "n_work", "n_slots", "stride", "_host", "_put")
+    __slots__ = ("plan", "n", "n_work", "n_slots", "stride", "_host", "_put")
 
     rows = property(lambda self: self._put(self._host[0]))
     indptr = property(lambda self: self._put(self._host[1]))
@@ -226,9 +220,9 @@ class MI355XBackend:
         # The split-K workspace. A pool sized by sizing.plan_kv_pool passes its
         # workspace_bytes here, so no batch within that plan's limits ever
         # allocates at run time; a plan that needs more grows it.
+        self._planned: _Plan | None = None
         self._set_workspace(torch.zeros(decode_workspace_bytes, dtype=torch.uint8,
                                         device=self.device))
-        self._planned: _Plan | None = None
         self._slot_cache: tuple[BatchMeta, torch.Tensor] | None = None
         self._pending: _Pending | None = None
         self.n_plans = 0
@@ -292,6 +286,8 @@ class MI355XBackend:
         self._workspace = ws
         self._ws_ptr = ws.data_ptr() if ws.numel() else None
         self._ws_bytes = ws.numel()
+        if self._planned is not None:   # described again, with this workspace
+            self._planned.batch = self._planned.batch_ptr = None
         # leading bytes known to be zero between launches (a new workspace
         # is zero-filled)
         self._ws_zero = ws.numel()
@@ -395,6 +391,13 @@ class MI355XBackend:
                 pend.kver, pend.vver = k._version, v._version
                 self._pending = pend
                 return
+            if p is not None and p.n_tokens == tokens and tokens:
+                rc = self._lib.pkv_append_batch(
+                    p.batch_ptr or self._describe(p), self._k_ptr[layer_idx],
+                    self._v_ptr[layer_idx], k.data_ptr(), v.data_ptr(), stream)
+                if rc:
+                    _native.check(rc, "append_kv")
+                return
         self._launch_append(layer_idx, k, v, self._slots_for(meta), stream)
 
     def _slots_for(self, meta: BatchMeta) -> torch.Tensor:
@@ -471,36 +474,12 @@ class MI355XBackend:
         kp = self._k_ptr[layer_idx]
         vp = self._v_ptr[layer_idx]
         self.n_runs += 1
-        if not p.use_prefill:
-            self._launch_decode(q, out, kp, vp, p.ptrs, p.n_seqs, p.n_work, p.n_slots,
-                                p.stride, scale, stream, pend if fused else None)
-        else:
-            cu_q, indptr, indices, kv_lens, bidx, plan = p.pre_ptrs
-            batch = (q.data_ptr(), out.data_ptr(), kp, vp, self.num_blocks, cu_q, indptr, indices,
-                     kv_lens, bidx, p.n_seqs, p.n_tokens, self.n_heads, self.n_kv_heads,
-                     self.head_dim, self.block_size, float(scale), self._code, plan, p.n_work,
-                     self.q_tile)
-            d = p.dec
-            if d is None:
-                rc = self._lib.pkv_attend_prefill(*batch, self._status_ptr, stream)
-            else:
-                rc = self._lib.pkv_attend_mixed(*batch, d.ptr, d.n, d.n_work, d.n_slots, d.stride,
-                                                self._ws_ptr, self._ws_bytes, self._status_ptr,
-                                                stream)
-            _native.check(rc, "attend (prefill)")
+        rc = self._lib.pkv_attend_batch(
+            p.batch_ptr or self._describe(p), q.data_ptr(), out.data_ptr(), kp, vp, float(scale),
+            pend.k.data_ptr() if fused else None, pend.v.data_ptr() if fused else None, stream)
+        if rc:
+            _native.check(rc, "attend (prefill)" if p.use_prefill else "attend (decode)")
         return out
-
-    def _launch_decode(self, q, out, kp, vp, ptrs, n_seqs, n_work, n_slots, stride, scale,
-                       stream, pend) -> None:
-        """``ptrs``: device addresses of (indptr, indices, kv_lens, plan, slots)."""
-        indptr, indices, kv_lens, plan, slots = ptrs
-        rc = self._lib.pkv_attend_decode(
-            q.data_ptr(), out.data_ptr(), kp, vp, self.num_blocks, indptr, indices, kv_lens,
-            n_seqs, self.n_heads, self.n_kv_heads, self.head_dim, self.block_size,
-            float(scale), self._code, plan, n_work, n_slots, stride,
-            pend.k.data_ptr() if pend else None, pend.v.data_ptr() if pend else None,
-            slots if pend else None, self._ws_ptr, self._ws_bytes, self._status_ptr, stream)
-        _native.check(rc, "attend (decode)")
 
     # -- planning ---------------------------------------------------------------
 
@@ -598,12 +577,28 @@ class MI355XBackend:
         p.bidx = self._dev_i32(meta.batch_indices)
         p.slots = (self._dev_i32(meta.slot_mapping) if meta.slot_mapping is not None
                    else None)
-        p.ptrs = _decode_ptrs(p.indptr, p.indices, p.kv_lens, p.plan, p.slots)
-        p.pre_ptrs = tuple(t.data_ptr() for t in (p.cu_q, p.indptr, p.indices, p.kv_lens, p.bidx,
-                                                  p.plan))
+        p.batch = p.batch_ptr = None
         self._planned = p
         self.n_plans += 1
         return p
+
+    def _describe(self, p: _Plan) -> int:
+        """Address of the plan's ``pkv_batch``: the arguments its launches share,
+        converted once instead of per layer."""
+        at = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
+        d = p.dec or p
+        p.batch = _native.Batch(
+            num_blocks=self.num_blocks, cu_query_lens=at(p.cu_q), kv_indptr=at(p.indptr),
+            kv_indices=at(p.indices), kv_lens=at(p.kv_lens), batch_indices=at(p.bidx),
+            slot_mapping=at(p.slots), prefill_plan=at(p.plan), decode_plan=at(d.plan),
+            workspace=self._ws_ptr, workspace_bytes=self._ws_bytes,
+            status_word=self._status_ptr, n_seqs=p.n_seqs, n_tokens=p.n_tokens, n_heads=self.n_heads,
+            n_kv_heads=self.n_kv_heads, head_dim=self.head_dim, page_size=self.block_size,
+            dtype=self._code, is_prefill=p.use_prefill, n_tiles=p.n_work, q_tile=self.q_tile,
+            n_decodes=p.dec.n if p.dec is not None else 0, n_work=d.n_work, n_slots=d.n_slots,
+            plan_stride=d.stride)
+        p.batch_ptr = C.addressof(p.batch)
+        return p.batch_ptr
 
     def _plan_decode(self, indptr32, indices32, kvl32, last32, n):
         """Host decode plan (pkv_plan_decode) plus a workspace large enough for it.
@@ -677,7 +672,6 @@ class MI355XBackend:
         at = (bins + 1) * d.stride - 8 * (np.arange(bins.shape[0]) - first + 1)
         plan[at + 7] = (plan[at + 7] & 1) | (rows[plan[at]] << 1)
         d.plan = self._upload(plan)
-        d.ptr = d.plan.data_ptr()
         d._host, d._put = host, self._upload
         return d
 

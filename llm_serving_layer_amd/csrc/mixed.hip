@@ -126,3 +126,39 @@ extern "C" int pkv_attend_mixed(const void* q, void* out, void* k_pool, void* v_
                            decode_plan, n_work, n_slots, plan_stride, nullptr, nullptr, nullptr,
                            workspace, workspace_bytes, status_word, stream);
 }
+
+static_assert(sizeof(pkv_batch) == 152, "the layout the Python binding fills");
+
+extern "C" int pkv_append_batch(const void* batch, void* k_pool, void* v_pool, const void* k,
+                                const void* v, void* stream) {
+  if (!batch) return fail(PKV_ERR_INVALID, "null batch");
+  const pkv_batch& b = *static_cast<const pkv_batch*>(batch);
+  return pkv_append_kv(k_pool, v_pool, b.num_blocks * b.page_size, k, v, b.slot_mapping,
+                       b.n_tokens, b.n_kv_heads, b.head_dim, b.dtype, b.status_word, stream);
+}
+
+extern "C" int pkv_attend_batch(const void* batch, const void* q, void* out, void* k_pool,
+                                void* v_pool, float scale, const void* k_new, const void* v_new,
+                                void* stream) {
+  if (!batch) return fail(PKV_ERR_INVALID, "null batch");
+  const pkv_batch& b = *static_cast<const pkv_batch*>(batch);
+  if (!b.is_prefill)
+    return pkv_attend_decode(q, out, k_pool, v_pool, b.num_blocks, b.kv_indptr, b.kv_indices,
+                             b.kv_lens, b.n_seqs, b.n_heads, b.n_kv_heads, b.head_dim,
+                             b.page_size, scale, b.dtype, b.decode_plan, b.n_work, b.n_slots,
+                             b.plan_stride, k_new, v_new, k_new ? b.slot_mapping : nullptr,
+                             b.workspace, b.workspace_bytes, b.status_word, stream);
+  if (k_new || v_new)
+    return fail(PKV_ERR_INVALID, "a fused append needs a batch of decodes only");
+  if (b.n_decodes > 0)
+    return pkv_attend_mixed(q, out, k_pool, v_pool, b.num_blocks, b.cu_query_lens, b.kv_indptr,
+                            b.kv_indices, b.kv_lens, b.batch_indices, b.n_seqs, b.n_tokens,
+                            b.n_heads, b.n_kv_heads, b.head_dim, b.page_size, scale, b.dtype,
+                            b.prefill_plan, b.n_tiles, b.q_tile, b.decode_plan, b.n_decodes,
+                            b.n_work, b.n_slots, b.plan_stride, b.workspace, b.workspace_bytes,
+                            b.status_word, stream);
+  return pkv_attend_prefill(q, out, k_pool, v_pool, b.num_blocks, b.cu_query_lens, b.kv_indptr,
+                            b.kv_indices, b.kv_lens, b.batch_indices, b.n_seqs, b.n_tokens,
+                            b.n_heads, b.n_kv_heads, b.head_dim, b.page_size, scale, b.dtype,
+                            b.prefill_plan, b.n_tiles, b.q_tile, b.status_word, stream);
+}
