@@ -174,7 +174,7 @@ __device__ __forceinline__ void merge_head(T* __restrict__ out, float* wts, int 
 //  * the waves share the output dims for PV: each walks all pages in order
 //    for its own dims (V in LDS), and merges those dims of a cut sequence.
 // One 1371-token sequence (5 pieces, 8 KV heads, 32 query heads, d 64): 16.4
-// us a launch in decode_kernel; 16 layers of such steps 271 -> 167 us.
+// us a launch in decode_kernel; 9.4 here; 16 layers of such steps 271 -> 157 us.
 template <typename T, int D, int G> struct PieceLds {
   static constexpr int CH = 20;                   // pages staged at a time: any piece of
                                                   // the default cut (17 + a folded tail)
@@ -545,7 +545,7 @@ template <int D> constexpr int kPieceWaves = D == 64 ? 3 : 1;
 
 // One piece a workgroup while those workgroups are all resident at once (768
 // at d = 64, 256 at d = 128), the streaming kernel beyond: at d = 64, us a
-// layer and piece against streaming, 40 workgroups 10.4 against 17.0, 480 13.9
+// layer and piece against streaming, 40 workgroups 9.8 against 17.0, 480 13.9
 // against 17.6, 1280 16.7 against 15.8; at d = 128, 144 12.6 against 17.6, 456
 // 19.0 against 19.3. Fewer than 256 workgroups' worth of bins means one piece
 // a bin (the plan makes as many bins as pieces until the grid is full).
