@@ -249,6 +249,9 @@ int pkv_attend_prefill(const void* q, void* out,
  * launch where neither fills the chip. prefill_plan covers the multi-token
  * sequences only; decode_plan is pkv_plan_decode's output over the n_decodes
  * one-token sequences, its items' rows set to their token rows of q and out.
+ * With n_decodes > 0 the geometry must have the fast decode path
+ * (pkv_decode_fast_path; else PKV_ERR_INVALID, nothing launched: run such a
+ * batch whole through pkv_attend_prefill) and q be 16-byte aligned.
  * No reference counterpart: the reference attends a mixed batch sequence by
  * sequence (serving/backends/paged_torch.py:280-485).
  */

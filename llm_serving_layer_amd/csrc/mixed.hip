@@ -97,6 +97,11 @@ extern "C" int pkv_attend_mixed(const void* q, void* out, void* k_pool, void* v_
                                 int32_t* status_word, void* stream) {
   int rc = check_geometry(n_heads, n_kv_heads, head_dim, page_size, dtype);
   if (rc) return rc;
+  // Without a plan-driven decode kernel the decode call would take the batch's
+  // first n_decodes sequences for the decodes.
+  if (n_decodes > 0 && !pkv_decode_fast_path(n_heads, n_kv_heads, head_dim, page_size, dtype, 1))
+    return fail(PKV_ERR_INVALID, "a mixed batch's decodes need the fast decode path "
+                "(see pkv_decode_fast_path)");
   const int32_t G = n_heads / n_kv_heads;
   const int32_t groups = n_kv_heads / heads_per_wg(n_kv_heads);
   const uintptr_t al = (uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pool | (uintptr_t)v_pool;
