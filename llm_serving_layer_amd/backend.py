@@ -517,6 +517,10 @@ class MI355XBackend:
             self._flush()
         if not (q.dtype is self.dtype and q.get_device() == di and q.is_contiguous()):
             q = self._as_pool(q)
+        if p.dec is not None and q.data_ptr() % 16 and not C.c_float(float(scale)).value > 0:
+            # such a scale sends the chunks to the generic kernel, which takes
+            # any address; the decode kernel reads 16 bytes at a time
+            q = q.clone()
         out = torch.empty_like(q)
         kp = self._k_ptr[layer_idx]
         vp = self._v_ptr[layer_idx]

@@ -95,3 +95,26 @@ def test_decodes_of_a_mixed_batch_read_and_write_their_token_rows(n_decode):
     alone = make_meta(seqs[1:-1], [1] * n_decode, 16, device=DEV)
     assert torch.equal(bk.attend(q[7:7 + n_decode], 0, 0.125, alone), out[7:7 + n_decode])
     bk.check_device_errors()
+
+
+@pytest.mark.parametrize("scale", [-0.125, 0.0, 1e-50])
+def test_a_mixed_batch_takes_q_at_any_address_where_its_chunks_do(scale):
+    """A scale that is not positive in fp32 runs the chunks on the generic
+    kernel, so a q that starts 2 bytes into its storage is served, decodes
+    included; with a positive scale it is refused."""
+    print(f"mixed unaligned q scale={scale}", flush=True)
+    bk = MI355XBackend(1, 64, 16, 2, 8, 64, device=DEV)
+    alloc = BlockAllocator(64, 16)
+    seqs = [SequenceBlocks(alloc, seq_id=i) for i in range(3)]
+    grow_and_assemble(seqs, [30, 5, 300], 16)
+    meta = grow_and_assemble(seqs, [1, 20, 1], 16, device=DEV)
+    g = torch.Generator(device=DEV).manual_seed(8)
+    bk.k_pool[0].normal_(generator=g)
+    bk.v_pool[0].normal_(generator=g)
+    q = torch.randn(22 * 8 * 64 + 1, generator=g, device=DEV).half()[1:].view(22, 8, 64)
+    assert q.is_contiguous() and q.data_ptr() % 16
+    out = bk.attend(q, 0, scale, meta)
+    assert bk._planned.dec is not None and torch.isfinite(out).all()
+    assert torch.equal(out, bk.attend(q.clone(), 0, scale, meta))
+    with pytest.raises(ValueError, match="16-byte aligned"):
+        bk.attend(q, 0, 0.125, meta)
