@@ -76,34 +76,33 @@ __device__ __forceinline__ int swz(int row, int e) {
 }
 
 // NL loads of 16 bytes a lane straight to LDS: load k from range `rs` at byte
-// offset v[k] + k * step to LDS bytes lds + 1024 k + 16 * lane .. + 15. Written
-// in asm so that only the kernel's own waits cover them: where the compiler
-// cannot tell an LDS ring's tiles apart, it waits for every load in flight
-// before each tile read. No vector register is written; the no-ops cover
+// offset v[k] to LDS bytes lds + 1024 k + 16 * lane .. + 15. The whole offset
+// is the lane's: a scalar offset is documented as outside the range check.
+// Written in asm so that only the kernel's own waits cover them: where the
+// compiler cannot tell an LDS ring's tiles apart, it waits for every load in
+// flight before each tile read. No vector register is written; the no-ops cover
 // scalar registers written just before; m0, which the compiler may use, is put
 // back.
 template <int NL>
-__device__ __forceinline__ void load_to_lds(u32x4 rs, const uint32_t* v, uint32_t step,
-                                            uint32_t lds) {
+__device__ __forceinline__ void load_to_lds(u32x4 rs, const uint32_t* v, uint32_t lds) {
   static_assert(NL == 2 || NL == 4, "a page of 2 or 4 KiB");
   uint32_t m0;
   if constexpr (NL == 2)
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 4\n\t"
                  "buffer_load_dwordx4 %1, %3, 0 offen lds\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %2, %3, %6 offen lds\n\ts_mov_b32 m0, %0"
+                 "buffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
                  : "=&s"(m0)
-                 : "v"(v[0]), "v"(v[1]), "s"(rs), "s"(lds), "s"(lds + 1024), "s"(step)
+                 : "v"(v[0]), "v"(v[1]), "s"(rs), "s"(lds), "s"(lds + 1024)
                  : "memory");
   else
     asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %6\n\ts_nop 4\n\t"
                  "buffer_load_dwordx4 %1, %5, 0 offen lds\n\ts_mov_b32 m0, %7\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %2, %5, %10 offen lds\n\ts_mov_b32 m0, %8\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %3, %5, %11 offen lds\n\ts_mov_b32 m0, %9\n\ts_nop 0\n\t"
-                 "buffer_load_dwordx4 %4, %5, %12 offen lds\n\ts_mov_b32 m0, %0"
+                 "buffer_load_dwordx4 %2, %5, 0 offen lds\n\ts_mov_b32 m0, %8\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %3, %5, 0 offen lds\n\ts_mov_b32 m0, %9\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %4, %5, 0 offen lds\n\ts_mov_b32 m0, %0"
                  : "=&s"(m0)
                  : "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "s"(rs), "s"(lds),
-                   "s"(lds + 1024), "s"(lds + 2048), "s"(lds + 3072), "s"(step), "s"(2 * step),
-                   "s"(3 * step)
+                   "s"(lds + 1024), "s"(lds + 2048), "s"(lds + 3072)
                  : "memory");
 }
 // The buffer resource of ws_rsrc as the four words load_to_lds takes.

@@ -146,9 +146,10 @@ __device__ __forceinline__ void prefill_tile(
   constexpr int RPI = 64 / CPR;                  // rows of a wave load
   uint32_t voff[LPT];
 #pragma unroll
-  for (int k = 0; k < LPT; ++k) {                // (rows k * RPI: in the scalar offset)
-    const int lc = ((lane % CPR) ^ xr(k * RPI + lane / CPR)) & 7 | ((lane % CPR) & ~7);
-    voff[k] = (uint32_t)(lane / CPR) * rowbytes + (uint32_t)(h * RB + lc * 16);
+  for (int k = 0; k < LPT; ++k) {
+    const int rr = k * RPI + lane / CPR;
+    const int lc = ((lane % CPR) ^ xr(rr)) & 7 | ((lane % CPR) & ~7);
+    voff[k] = (uint32_t)rr * rowbytes + (uint32_t)(h * RB + lc * 16);
   }
   auto load_id = [&](int t) {   // this wave's page id for tile t
     return __builtin_amdgcn_readfirstlane(kv_indices[pbase + min(2 * t + wpage, npages - 1)]);
@@ -164,7 +165,7 @@ __device__ __forceinline__ void prefill_tile(
     load_to_lds<LPT>(
         raw_rsrc(reinterpret_cast<const char*>(wpool) + (uint64_t)pid * pagebytes,
                  live_rows > 0 ? (uint32_t)live_rows * rowbytes : 0u),
-        voff, RPI * rowbytes, lds_address(dst) + wdst);
+        voff, lds_address(dst) + wdst);
   };
 
   // O^T accumulators: o[dh][rr] = O[row][32 dh + 8 (rr / 4) + 4 g + rr % 4].
