@@ -517,16 +517,18 @@ class MI355XBackend:
             self._flush()
         if not (q.dtype is self.dtype and q.get_device() == di and q.is_contiguous()):
             q = self._as_pool(q)
-        if p.dec is not None and q.data_ptr() % 16 and not C.c_float(float(scale)).value > 0:
+        q_ptr = q.data_ptr()
+        if q_ptr % 16 and p.dec is not None and not C.c_float(float(scale)).value > 0:
             # such a scale sends the chunks to the generic kernel, which takes
             # any address; the decode kernel reads 16 bytes at a time
             q = q.clone()
+            q_ptr = q.data_ptr()
         out = torch.empty_like(q)
         kp = self._k_ptr[layer_idx]
         vp = self._v_ptr[layer_idx]
         self.n_runs += 1
         rc = self._lib.pkv_attend_batch(
-            p.batch_ptr or self._describe(p), q.data_ptr(), out.data_ptr(), kp, vp, float(scale),
+            p.batch_ptr or self._describe(p), q_ptr, out.data_ptr(), kp, vp, float(scale),
             pend.k.data_ptr() if fused else None, pend.v.data_ptr() if fused else None, stream)
         if rc:
             _native.check(rc, "attend (prefill)" if p.use_prefill else "attend (decode)")
