@@ -92,7 +92,9 @@ int pkv_append_kv(void* k_pool, void* v_pool, int64_t num_slots,
  * a larger one may set it to a row of the larger one's arrays)} at the end of the block, item i at 8 (i + 1) ints
  * before the next block -- pieces of cut sequences before their last, whole
  * sequences, then the last pieces; then 64 zero ints. *plan_stride_out is at
- * least 68.
+ * least 68, and a multiple of 8 if every bin holds one item, 4 more than one
+ * otherwise: by it (and the sizes) a launch picks the kernel for few pieces or
+ * the one that streams bins. Either serves any plan, with the same bits.
  * *plan_needed (if not NULL) receives the ints required; a plan larger than
  * plan_capacity returns PKV_ERR_CAPACITY and writes nothing else.
  * *n_work_out is the grid size (workgroups), *n_slots_out the partial slots

@@ -73,6 +73,7 @@
 // the result is exactly "append, then attend" (the caller guarantees that no
 // other sequence of the launch reads that slot).
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <queue>
 #include <vector>
@@ -722,10 +723,25 @@ static void launch(const void* q, void* out, void* kp, void* vp, int64_t nb,
                        lds, s, (const T*)q, (T*)out, (T*)kp, (T*)vp, nb, plan, stride, Hkv, sl2,
                        (const T*)kn, (const T*)vn, slots, po, pml, o_bytes, ml_bytes, cnt, status);
   };
-  if (few_pieces(n_work, Hkv, D))
+  if (few_pieces(n_work, stride, Hkv, D))
     go(decode_piece_kernel<T, D, G>, Hkv, 256, 0);
   else
     go(decode_kernel<T, D, G>, groups, hgw * 64, decode_lds_bytes<T, D, G>(hgw));
+}
+
+constexpr int kMaxDevices = 64;
+
+int compute_units() {
+  static std::atomic<int> known[kMaxDevices];   // asked once per device
+  int dev = -1, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  cus = known[dev].load(std::memory_order_relaxed);
+  if (cus <= 0) {
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return 0;
+    known[dev].store(cus, std::memory_order_relaxed);
+  }
+  return cus;
 }
 
 // Workgroups of decode_kernel<T, D, G> that stay resident on one compute
@@ -806,10 +822,8 @@ extern "C" int pkv_decode_workgroups(int32_t n_heads, int32_t n_kv_heads, int32_
   if (n_kv_heads <= 0 || n_heads % n_kv_heads || per_cu <= 0) return 0;
   const Variant v = fast_variant(dtype, n_kv_heads, head_dim, n_heads / n_kv_heads, 16);
   if (!v.resident) return 0;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
+  const int cus = compute_units();
+  if (cus <= 0) return 0;
   const int fit = v.resident(n_kv_heads);
   return cus * std::min(per_cu, fit);
 }
@@ -902,6 +916,8 @@ extern "C" int pkv_plan_decode(const int32_t* kv_indptr, const int32_t* kv_indic
   for (int64_t b = 0; b < bins; ++b)
     stride = std::max<int64_t>(stride, kHdrInts + ((bin_pages[b] + 3) & ~3LL) +
                                            kItemInts * (int64_t)bin_count[b + 1]);
+  // (it was a multiple of 4: which one says what few_pieces asks)
+  if ((stride % 8 == 0) != (bins == (int64_t)n_items)) stride += 4;
   // in a bin: pieces before a cut sequence's last, whole sequences, then last
   // pieces, each in dealing order (longest first): a stable sort by (bin, role)
   for (int64_t b = 0; b < bins; ++b) bin_count[b + 1] += bin_count[b];
@@ -1054,7 +1070,6 @@ static int attend_decode(const void* q, void* out, void* k_pool, void* v_pool,
 // hipGetSymbolAddress and only that address is passed to kernels.
 static __device__ __align__(256) unsigned char scratch[PKV_DECODE_SCRATCH_BYTES];
 
-constexpr int kMaxDevices = 64;
 static void* g_scratch_ptr[kMaxDevices];
 static std::mutex g_scratch_mu;
 

@@ -228,7 +228,7 @@ __device__ __forceinline__ void decode_piece(
   const __amdgpu_buffer_rsrc_t ro = ws_rsrc(part_o, o_bytes);
   const __amdgpu_buffer_rsrc_t rm = ws_rsrc(part_ml, ml_bytes);
 
-  // One item, unless the plan was made for fewer workgroups than fit. (The
+  // One item where the launch follows few_pieces; any plan is served. (The
   // count, the item and its words come in one round trip; the slot below a
   // bin's last item still lies inside its plan block.)
   const int n_items = bp[0];
@@ -543,15 +543,28 @@ __device__ __forceinline__ void decode_piece(
 // d = 64, one at d = 128 (what their LDS allows).
 template <int D> constexpr int kPieceWaves = D == 64 ? 3 : 1;
 
-// One piece a workgroup while those workgroups are all resident at once (768
-// at d = 64, 256 at d = 128), the streaming kernel beyond: at d = 64, us a
-// layer and piece against streaming, 40 workgroups 9.8 against 17.0, 480 13.9
-// against 17.6, 1280 16.7 against 15.8; at d = 128, 144 12.6 against 17.6, 456
-// 19.0 against 19.3. Fewer than 256 workgroups' worth of bins means one piece
-// a bin (the plan makes as many bins as pieces until the grid is full).
-static inline bool few_pieces(int32_t n_work, int32_t Hkv, int32_t D) {
-  const int64_t bins = n_work / (Hkv / heads_per_wg(Hkv));
-  return n_work < 256 && bins * Hkv <= (D == 64 ? 768 : 256);
+// Whether every bin of a plan holds one piece, which pkv_plan_decode says in
+// the stride: a multiple of 8 ints then, 4 more than one otherwise.
+static inline bool one_piece_bins(int32_t plan_stride) { return plan_stride % 8 == 0; }
+
+// Compute units of the current device, 0 if it cannot be asked.
+int compute_units();
+
+// One piece a workgroup where no bin holds more than one and those workgroups
+// are all resident at once (3 a compute unit at d = 64, 1 at d = 128; 768 and
+// 256 here), the streaming kernel beyond: at d = 64, us a layer and piece
+// against streaming, 40 workgroups 9.8 against 17.0, 480 13.9 against 17.6,
+// 1280 16.7 against 15.8; at d = 128, 144 12.6 against 17.6, 456 19.0 against
+// 19.3. Bins of several pieces always stream: the piece kernel would take them
+// one after another with no page in flight between them (1024 sequences of 16
+// to 64 tokens in 32 bins of 8 heads: 113 us against 83). From a streaming
+// workgroup a compute unit on, batches stream too, which matters to 1, 2 and odd
+// numbers of KV heads: 200 pieces of 1 head 6.5 us (pieces), 300 11.3
+// (streaming), where the piece kernel would take 6.9.
+static inline bool few_pieces(int32_t n_work, int32_t plan_stride, int32_t Hkv, int32_t D) {
+  if (!one_piece_bins(plan_stride)) return false;
+  const int64_t cus = compute_units(), bins = n_work / (Hkv / heads_per_wg(Hkv));
+  return n_work < cus && bins * Hkv <= cus * (D == 64 ? 3 : 1);
 }
 
 // The parts of a decode workspace.

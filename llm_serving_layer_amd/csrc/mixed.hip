@@ -71,11 +71,6 @@ static MixedFn mixed_fn(int32_t dtype, int32_t D, int32_t G) {
   return nullptr;
 }
 
-// Prefill workgroups up to which one launch takes both kinds: one a compute
-// unit. Beyond, the tiles fill the chip by themselves, and this kernel's
-// registers and LDS (those of the larger body) would cost them occupancy.
-constexpr int64_t kMixedPrefillBlocks = 256;
-
 int split_workspace(void* workspace, int64_t workspace_bytes, int32_t n_seqs, int32_t n_slots,
                     int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, DecodeWorkspace* w);
 int check_geometry(int32_t Hq, int32_t Hkv, int32_t D, int32_t ps, int32_t dtype);
@@ -106,11 +101,14 @@ extern "C" int pkv_attend_mixed(const void* q, void* out, void* k_pool, void* v_
   const int32_t groups = n_kv_heads / heads_per_wg(n_kv_heads);
   const uintptr_t al = (uintptr_t)q | (uintptr_t)out | (uintptr_t)k_pool | (uintptr_t)v_pool;
   MixedFn fn = page_size == 16 ? mixed_fn(dtype, head_dim, G) : nullptr;
+  // One launch takes both kinds up to one prefill workgroup a compute unit.
+  // Beyond, the tiles fill the chip by themselves, and the joint kernel's
+  // registers and LDS (those of the larger body) would cost them occupancy.
   if (fn && scale > 0.f && prefill_plan && n_tiles > 0 && q_tile == kPrefillRows / G &&
-      (int64_t)n_tiles * n_kv_heads <= kMixedPrefillBlocks && decode_plan && n_decodes > 0 &&
+      (int64_t)n_tiles * n_kv_heads <= compute_units() && decode_plan && n_decodes > 0 &&
       n_work > 0 && n_work % groups == 0 && n_slots >= 0 &&
       plan_stride >= kHdrInts + kStageMax * kItemInts &&
-      few_pieces(n_work, n_kv_heads, head_dim) && al % 16 == 0) {
+      few_pieces(n_work, plan_stride, n_kv_heads, head_dim) && al % 16 == 0) {
     MixedArgs a{q, out, k_pool, v_pool, num_blocks, cu_query_lens, kv_indptr, kv_indices, kv_lens,
                 n_kv_heads, scale * kLog2e, prefill_plan, n_tiles, decode_plan, n_work / groups,
                 plan_stride, {}, status_word};

@@ -146,6 +146,8 @@ def plan_decode(kv_lens, part_pages, workgroups=512, n_kv_heads=8, ps=16, indice
     heads_per_wg = 4 if n_kv_heads % 4 == 0 else 2 if n_kv_heads % 2 == 0 else 1
     n_bins = nw.value // (n_kv_heads // heads_per_wg)
     assert need.value == n_bins * S + 64 and not buf[n_bins * S:need.value].any()
+    # the stride says whether every bin holds one item
+    assert S % 4 == 0 and (S % 8 == 0) == all(buf[b * S] == 1 for b in range(n_bins))
     bins = []
     for b in range(n_bins):
         blk = buf[b * S:(b + 1) * S]
@@ -164,6 +166,33 @@ def plan_decode(kv_lens, part_pages, workgroups=512, n_kv_heads=8, ps=16, indice
         assert pos == n_pg
         bins.append(items)
     return indptr, bins, nw.value, ns.value
+
+
+def takes_pieces(plan, n_kv_heads: int, head_dim: int) -> bool:
+    """Whether a launch of this decode plan (``n_work``, ``stride``) runs the
+    small-batch kernel, a workgroup per piece and KV head; the streaming kernel
+    runs it otherwise. The rule of the dispatch, restated."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    heads_per_wg = 4 if n_kv_heads % 4 == 0 else 2 if n_kv_heads % 2 == 0 else 1
+    bins = plan.n_work // (n_kv_heads // heads_per_wg)
+    return (plan.stride % 8 == 0 and plan.n_work < cus
+            and bins * n_kv_heads <= cus * (3 if head_dim == 64 else 1))
+
+
+def other_stride(backend, bins: int) -> None:
+    """Lay the backend's current decode plan out 4 ints a bin wider, which
+    turns what its stride says (one item a bin, or several): launches then pick
+    the other decode kernel, for the same work."""
+    p = backend._planned
+    plan, old = p.plan.cpu().numpy(), p.stride
+    wide = np.zeros(plan.shape[0] + 4 * bins, dtype=np.int32)
+    for b in range(bins):
+        block = plan[b * old:(b + 1) * old]
+        at, words = b * (old + 4), old - 8 * int(block[0])
+        wide[at:at + words] = block[:words]
+        wide[at + words + 4:at + old + 4] = block[words:]
+    p.plan, p.stride = torch.from_numpy(wide).to(p.plan.device), old + 4
+    p.batch = p.batch_ptr = None          # described again at the next launch
 
 
 def meta_to_device(meta: BatchMeta, device, mirror: bool = True) -> BatchMeta:

@@ -24,7 +24,7 @@ from llm_serving_layer_amd.backend import DEFAULT_PART_PAGES, MI355XBackend
 from oracle import PagedTorchOracle
 
 from ._util import (assert_attention_close, fragmented_allocator, grow_and_assemble,
-                    lognormal_lengths, make_meta, meta_to_device)
+                    lognormal_lengths, make_meta, meta_to_device, takes_pieces)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -151,19 +151,21 @@ def test_split_k_and_packed_items_other_geometries(geom):
         plan = p.gpu._planned
         assert plan.n_slots > 0, "expected cut sequences"
         assert plan.n_work // (n_kv // min(n_kv, 4)) < len(lens), "expected several items per bin"
+        assert not takes_pieces(plan, n_kv, d)
 
 
 @pytest.mark.parametrize("geom", [(8, 32, 64), (1, 8, 64), (2, 32, 128)])
 def test_merge_bits_do_not_depend_on_which_wave_merges(geom):
     """With one bin, every piece of a cut sequence runs before its last piece
     in the same wave, so the last piece always merges with its own partial
-    from registers; with many bins whichever piece arrives last merges from
-    stored partials. The outputs must be the same bits."""
+    from registers; with more bins whichever piece arrives last merges from
+    stored partials, and with a bin for every piece the small-batch kernel runs
+    them. The outputs must be the same bits."""
     n_kv, n_heads, d = geom
     print(f"merge paths geom={geom}", flush=True)
     groups = n_kv // min(n_kv, 4)
     outs = []
-    for wgs in (groups, 64 * groups):
+    for wgs in (groups, 8 * groups, 64 * groups):
         p = Pair(1, 512, 16, n_kv, n_heads, d, part_pages=2, decode_workgroups=wgs)
         p.poison(6)
         alloc, _keep = fragmented_allocator(512, 16)
@@ -172,8 +174,9 @@ def test_merge_bits_do_not_depend_on_which_wave_merges(geom):
             s.append(n)
         res = p.step(grow_and_assemble(seqs, [1] * 6, 16), 30)
         check(res, f"workgroups {wgs}")
+        assert takes_pieces(p.gpu._planned, n_kv, d) == (wgs == 64 * groups)
         outs.append(res[0][1].cpu())
-    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
 
 
 def _shared_prefix_batch(alloc, n_seqs, prefix_tokens):
@@ -679,6 +682,7 @@ def test_packed_short_sequences_vs_oracle(part_pages, workgroups):
         check(p.step(meta, 10 + step), f"packed decode step {step}")
         plan = p.gpu._planned
         assert plan.n_work // 2 < len(lens), "expected several sequences per bin"
+        assert not takes_pieces(plan, 8, 64)
 
 
 def test_packed_sequence_equals_solo_bitwise():
@@ -702,6 +706,7 @@ def test_packed_sequence_equals_solo_bitwise():
         s.append(1)
     packed = bk.attend(q[:-1], 0, 0.125, make_meta(seqs[:-1], [1] * len(lens), 16, device=DEV))
     assert bk._planned.n_slots == 0 and bk._planned.n_work == 2, "expected one bin"
+    assert not takes_pieces(bk._planned, 8, 64)
     mixed = bk.attend(q, 0, 0.125, make_meta(seqs, [1] * len(seqs), 16, device=DEV))
     assert bk._planned.n_slots > 0, "expected the long sequence to be split"
     for i in range(len(lens)):
@@ -758,3 +763,4 @@ def test_packed_decode_other_geometries(geom, dtype):
     check(p.step(grow_and_assemble(seqs, lens, 16), 1), "history", tol, rtol)
     check(p.step(grow_and_assemble(seqs, [1] * len(lens), 16), 2), "packed step", tol, rtol)
     assert p.gpu._planned.n_work < len(lens), "several sequences per bin"
+    assert not takes_pieces(p.gpu._planned, n_kv, d)

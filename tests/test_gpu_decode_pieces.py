@@ -1,8 +1,9 @@
 """
 The two decode kernels (csrc/decode.hip) give one result: a sequence's output
 has the same bits whether its batch is small (a workgroup per piece and KV
-head) or large (bins of pieces streamed by resident workgroups), with the
-step's rows appended inside the launch, at the sizes where the small-batch
+head) or large (bins of pieces streamed by resident workgroups), and whether
+its bin holds one piece or many, with the step's rows appended inside the
+launch, at the sizes where the small-batch
 kernel can go wrong: one row, page edges, the pages its four waves share, its
 chunks of 20 pages and their remainders, every group size, and non-finite
 values in the unused rows of a last page.
@@ -16,7 +17,7 @@ import torch
 from llm_serving_layer_amd import BlockAllocator, SequenceBlocks
 from llm_serving_layer_amd.backend import MI355XBackend
 
-from ._util import grow_and_assemble, make_meta
+from ._util import grow_and_assemble, make_meta, other_stride, takes_pieces
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -55,7 +56,7 @@ def test_small_and_large_batches_give_the_same_bits(n_heads, d, dtype, part_page
     meta = grow_and_assemble(seqs, [1] * len(lens), 16, device=DEV)
     big.append_kv(0, kn, vn, meta)
     want = big.attend(q, 0, d ** -0.5, meta)
-    assert big._planned.n_work >= 256
+    assert big._planned.n_work >= 256 and not takes_pieces(big._planned, 1, d)
     assert torch.isfinite(want).all()
     for at in range(0, len(lens), 26):
         part = slice(at, min(at + 26, len(lens)))
@@ -64,7 +65,7 @@ def test_small_and_large_batches_give_the_same_bits(n_heads, d, dtype, part_page
         meta = grow_and_assemble(seqs[part], [1] * len(seqs[part]), 16, device=DEV)
         few.append_kv(0, kn[part], vn[part], meta)
         got = few.attend(q[part], 0, d ** -0.5, meta)
-        assert few._planned.n_work < 256
+        assert takes_pieces(few._planned, 1, d)
         assert torch.equal(got, want[part]), f"sequences from {at}"
     assert torch.equal(few.k_pool[0].view(torch.int16), big.k_pool[0].view(torch.int16))
     assert torch.equal(few.v_pool[0].view(torch.int16), big.v_pool[0].view(torch.int16))
@@ -118,3 +119,57 @@ def test_a_mixed_batch_takes_q_at_any_address_where_its_chunks_do(scale):
     assert torch.equal(out, bk.attend(q.clone(), 0, scale, meta))
     with pytest.raises(ValueError, match="16-byte aligned"):
         bk.attend(q, 0, 0.125, meta)
+
+
+@pytest.mark.parametrize("bins", [None, 1, 5])
+@pytest.mark.parametrize("n_kv, n_heads, d, dtype, part_pages", [
+    (8, 32, 64, torch.float16, 2), (8, 8, 64, torch.bfloat16, 5), (4, 8, 64, torch.bfloat16, 17),
+    (1, 16, 64, torch.bfloat16, 3), (2, 16, 64, torch.float16, 64), (1, 1, 128, torch.bfloat16, 3),
+    (2, 4, 128, torch.float16, 5), (1, 4, 128, torch.bfloat16, 17), (2, 16, 128, torch.bfloat16, 2),
+    (1, 16, 128, torch.float16, 5)])
+def test_either_kernel_serves_any_plan_with_the_same_bits(bins, n_kv, n_heads, d, dtype,
+                                                          part_pages):
+    """One plan through both kernels, with one piece a bin and with many (the
+    streaming kernel's item slots refilled, its output and row rings filled and
+    flushed, deferred arrivals, merges by the last arriver and by a last piece
+    with its own partial in registers), the step's rows appended in the launch.
+    Bins of several pieces stream."""
+    print(f"one plan, two kernels n_kv={n_kv} heads={n_heads} d={d} {dtype} bins={bins}",
+          flush=True)
+    lens = [0, 1, 15, 16, 17, 47, 48, 80, 303] + [3 * i for i in range(20)] + [500]
+    if bins is None:                   # few enough for a workgroup a piece and head
+        lens = lens[1:6] + [90]
+    groups = n_kv // min(n_kv, 4)
+    alloc = BlockAllocator(256, 16)
+    seqs = [SequenceBlocks(alloc, seq_id=i) for i in range(len(lens))]
+    for s, n in zip(seqs, lens):
+        s.append(n)
+    g = torch.Generator(device=DEV).manual_seed(9)
+    rand = lambda *s: torch.randn(s, generator=g, device=DEV).to(dtype)  # noqa: E731
+    bks = [MI355XBackend(1, 256, 16, n_kv, n_heads, d, device=DEV, dtype=dtype,
+                         part_pages=part_pages,
+                         decode_workgroups=None if bins is None else bins * groups)
+           for _ in range(2)]
+    k, v = rand(256, 16, n_kv, d), rand(256, 16, n_kv, d)
+    for bk in bks:
+        bk.k_pool[0].copy_(k)
+        bk.v_pool[0].copy_(v)
+    n = len(lens)
+    for _ in range(2):
+        meta = grow_and_assemble(seqs, [1] * n, 16, device=DEV)
+        q, kn, vn = 2.0 * rand(n, n_heads, d), rand(n, n_kv, d), rand(n, n_kv, d)
+        outs, kinds = [], []
+        for i, bk in enumerate(bks):
+            bk.append_kv(0, kn, vn, meta)
+            assert bk._pending is not None, "the append rides in the launch"
+            p = bk._planned
+            if i:
+                other_stride(bk, p.n_work // groups)
+            kinds.append(takes_pieces(p, n_kv, d))
+            outs.append(bk.attend(q, 0, d ** -0.5, meta))
+        assert kinds == [bins is None, bins is not None]
+        assert torch.isfinite(outs[0]).all() and torch.equal(*outs)
+        for a, b in zip(*(bk.k_pool + bk.v_pool for bk in bks)):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    for bk in bks:
+        bk.check_device_errors()
