@@ -167,15 +167,9 @@ class _Plan:
 class _DecodeRows:
     """The one-token sequences of a mixed batch, run through the decode kernel:
     their decode plan as a batch of their own, whose items name their token
-    rows in the whole batch's q and out. The rest (rows, CSR, lengths) is on
-    the host until asked for: the decode kernel reads only the plan."""
+    rows in the whole batch's q and out (the plan is all the kernel reads)."""
 
-    __slots__ = ("plan", "n", "n_work", "n_slots", "stride", "_host", "_put")
-
-    rows = property(lambda self: self._put(self._host[0]))
-    indptr = property(lambda self: self._put(self._host[1]))
-    kv_lens = property(lambda self: self._put(self._host[2]))
-    indices = property(lambda self: self._put(self._host[3]))
+    __slots__ = ("plan", "n", "n_work", "n_slots", "stride")
 
 
 class _Pending:
@@ -711,11 +705,10 @@ class MI355XBackend:
         page_ix = np.repeat(indptr[dec] - sub_ptr[:-1], npg) + np.arange(int(sub_ptr[-1]))
         i32 = lambda a: np.ascontiguousarray(a, dtype=np.int32)  # noqa: E731
         rows = cu[dec]
-        host = (rows.astype(np.int64), i32(sub_ptr), i32(kvl[dec]), i32(indices[page_ix]))
         d = _DecodeRows()
         d.n = int(dec.shape[0])
-        plan, d.n_work, d.n_slots, d.stride = self._plan_decode(host[1], host[3], host[2],
-                                                                i32(last[dec]), d.n)
+        plan, d.n_work, d.n_slots, d.stride = self._plan_decode(
+            i32(sub_ptr), i32(indices[page_ix]), i32(kvl[dec]), i32(last[dec]), d.n)
         # item i of a bin: 8 (i + 1) ints before the bin's end; its sequence
         # first, its flags (last-page bit, then the row) last
         blocks = plan[:plan.shape[0] // d.stride * d.stride].reshape(-1, d.stride)
@@ -725,7 +718,6 @@ class MI355XBackend:
         at = (bins + 1) * d.stride - 8 * (np.arange(bins.shape[0]) - first + 1)
         plan[at + 7] = (plan[at + 7] & 1) | (rows[plan[at]] << 1)
         d.plan = self._upload(plan)
-        d._host, d._put = host, self._upload
         return d
 
     def _upload(self, a: np.ndarray) -> torch.Tensor:

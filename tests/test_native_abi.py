@@ -276,7 +276,7 @@ def test_backend_plans_decode_and_prefill_through_the_library():
 def test_mixed_batch_plans_its_decodes_for_the_decode_kernel():
     """Prefill chunks beside one-token decodes: the prefill tiles cover only
     the multi-token sequences, and the one-token sequences form a decode
-    batch of their own (rows, CSR over their own pages, plan)."""
+    batch of their own, whose plan names their pages and their token rows."""
     from llm_serving_layer_amd import BlockAllocator, SequenceBlocks
 
     from ._util import grow_and_assemble
@@ -291,16 +291,23 @@ def test_mixed_batch_plans_its_decodes_for_the_decode_kernel():
     tiles = p.plan.reshape(-1, 4).numpy()
     assert set(tiles[:, 0]) == {1, 3}, "prefill tiles must skip the one-token sequences"
     d = p.dec
-    assert d.n == 2 and d.rows.tolist() == [0, 31]   # token rows of sequences 0 and 2
-    assert d.kv_lens.tolist() == [41, 8]
+    assert d.n == 2 and d.n_slots > 0
     indptr, indices = meta.kv_indptr.tolist(), meta.kv_indices.tolist()
-    want = indices[indptr[0]:indptr[1]] + indices[indptr[2]:indptr[3]]
-    assert d.indices.tolist() == want and d.indptr.tolist() == [0, 3, 4]
-    seqs_planned = set()
+    # what the decode kernel reads: each item's sequence of the sub-batch, its
+    # length, its token row in the whole batch (0 and 31), its pages in order
+    pages = {0: [], 1: []}
     for b in range(d.n_work // 2):
-        blk = d.plan[b * d.stride:(b + 1) * d.stride].numpy()
-        seqs_planned |= {int(blk[d.stride - 8 * (i + 1)]) for i in range(int(blk[0]))}
-    assert d.n_slots > 0 and seqs_planned == {0, 1}, "decode plan over the sub-batch"
+        blk = d.plan[b * d.stride:(b + 1) * d.stride].tolist()
+        at = 4
+        for i in range(blk[0]):
+            seq, n, tok0, kv, _, _, _, flags = blk[d.stride - 8 * (i + 1):][:8]
+            assert kv == [41, 8][seq] and flags >> 1 == [0, 31][seq]
+            assert (flags & 1) == (tok0 + 16 * n >= kv), "the last piece says so"
+            pages[seq] += [(tok0 // 16 + j, w & ((1 << 27) - 1))
+                           for j, w in enumerate(blk[at:at + n])]
+            at += n
+    assert sorted(pages[0]) == list(enumerate(indices[indptr[0]:indptr[1]]))
+    assert sorted(pages[1]) == list(enumerate(indices[indptr[2]:indptr[3]]))
 
 
 def test_decode_plan_falls_back_to_larger_pieces_past_2gib_of_partials():
