@@ -655,7 +655,7 @@ class MI355XBackend:
         ptr = lambda a: a.ctypes.data  # noqa: E731
         n_work, n_slots, stride = C.c_int32(), C.c_int32(), C.c_int32()
         needed = C.c_int64()
-        cap = 6 * self._decode_wgs + 2 * int(indptr32[-1]) + 24 * n + 128
+        cap = 10 * self._decode_wgs + 2 * int(indptr32[-1]) + 24 * n + 128
         counter_bytes = (4 * n * self.n_kv_heads + 255) // 256 * 256
         part_pages = self.part_pages
         while True:

@@ -558,9 +558,9 @@ int compute_units();
 // 19.3. Bins of several pieces always stream: the piece kernel would take them
 // one after another with no page in flight between them (1024 sequences of 16
 // to 64 tokens in 32 bins of 8 heads: 113 us against 83). From a streaming
-// workgroup a compute unit on, batches stream too, which matters to 1, 2 and odd
-// numbers of KV heads: 200 pieces of 1 head 6.5 us (pieces), 300 11.3
-// (streaming), where the piece kernel would take 6.9.
+// workgroup a compute unit on, batches stream too, which matters to numbers of
+// KV heads that 4 does not divide: 200 pieces of 1 head 6.5 us (pieces), 300
+// 11.3 (streaming), where the piece kernel would take 6.9.
 static inline bool few_pieces(int32_t n_work, int32_t plan_stride, int32_t Hkv, int32_t D) {
   if (!one_piece_bins(plan_stride)) return false;
   const int64_t cus = compute_units(), bins = n_work / (Hkv / heads_per_wg(Hkv));
