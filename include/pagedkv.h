@@ -89,8 +89,8 @@ int pkv_append_kv(void* k_pool, void* v_pool, int64_t num_slots,
  * of the sequence, its first slot, flags (bit 0: the piece holds the
  * sequence's last page; from bit 1: the sequence's row of q, out, k_new, v_new
  * and slot_mapping, its index as planned -- a caller whose batch is part of
- * a larger one may set it to a row of the larger one's arrays)} at the end of the block, item i at 8 (i + 1) ints
- * before the next block -- pieces of cut sequences before their last, whole
+ * a larger one may set it to a row of the larger one's arrays)} at the end of
+ * the block, item i at 8 (i + 1) ints before the next block -- pieces of cut sequences before their last, whole
  * sequences, then the last pieces; then 64 zero ints. *plan_stride_out is at
  * least 68, and a multiple of 8 if every bin holds one item, 4 more than one
  * otherwise: by it (and the sizes) a launch picks the kernel for few pieces or
